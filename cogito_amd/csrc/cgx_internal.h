@@ -26,6 +26,8 @@ enum { CGX_SLOT_IN0 = 0, CGX_SLOT_IN1, CGX_SLOT_IN2, CGX_SLOT_IN3,
        CGX_SLOT_WS2, CGX_SLOT_WS3, CGX_SLOT_WS4, CGX_SLOT_WS5, CGX_SLOT_WS6,
        CGX_NUM_SLOTS };
 void* cgx_scratch(int slot, size_t bytes);
+/* 1 while the library stream is being captured into a graph. */
+int cgx_is_capturing(void);
 /* Zero-initialised counters that kernels reset themselves after use. */
 unsigned int* cgx_counters(size_t count);
 /* Device view of a host-or-device argument: returns p itself when it is a
@@ -85,6 +87,12 @@ int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs, const ui
                   const float* scales_t, float smax, float* y, int ldy, int pro,
                   const float* nw, float eps, int epi, const float* stats_in, int nstat_in,
                   float* stats_out, const float* nw_next);
+/* Dispatch of plain products between the GEMM and the GEMV: whether M rows
+ * pay for the GEMM, the rows of one GEMM call, and whether its scratch is at
+ * hand (not under stream capture). */
+int cgk_gemm_int4_pays(int M, int K, int N, int gs);
+int cgk_gemm_int4_max_rows(int K, int N);
+int cgk_gemm_int4_ready(int M, int K, int N);
 int cgk_absmax(const float* s, size_t n, float* out_host);
 int cgk_gemv_mfma(const float* x, int ldx, int M, int K, int N, int gs, const uint8_t* w,
                   const float* scales_t, float* y, int ldy, int pro, const float* nw, float eps,

@@ -944,6 +944,14 @@ int launch_pe(const MfmaArgs& a, int T) {
 constexpr int kGemmWaves = 4;
 constexpr int kGemmTiles = 4;            // column tiles per wave
 constexpr int kGemmRowH = kChunkK + 8;   // LDS pitch (halfs) of an A row
+// 128-row chunks per first-level sum: the MFMA accumulators run over 512 k
+// values and are then added to the split's sums, so that few roundings happen
+// at a long sum's full magnitude (error against 64 bits, 4096 x 11008 at 509
+// rows: 4.7e-7 of the result in one chain, 1.9e-7 folded, 2.0e-7 in the GEMV;
+// for 3 % of the time, 114 -> 118 us).  Plain products only: the decoder's
+// layers keep one chain (two layers of the 7B shape at 256 rows: 610 us in one
+// chain, 644 folded).
+constexpr int kGemmFold = 4;
 
 struct GemmArgs {
     const float* x;           // [M][ldx]
@@ -967,7 +975,7 @@ struct GemmArgs {
     const float* nw_next;     // the next linear's RMSNorm weights, or nullptr
 };
 
-template <int RT, int NG, int PRO>
+template <int RT, int NG, int PRO, bool FOLD>
 __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
     constexpr int BM = 16 * RT;
     constexpr int RPT = BM / 8;                 // rows prepared per thread
@@ -1099,11 +1107,21 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     wload(c0, wb0);
 
-    f32x4 acc[kGemmTiles][RT];
+    f32x4 acc[kGemmTiles][RT], tot[kGemmTiles][RT];
 #pragma unroll
     for (int j = 0; j < kGemmTiles; j++)
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) acc[j][rt] = (f32x4)(0.0f);
+        for (int rt = 0; rt < RT; rt++) acc[j][rt] = tot[j][rt] = (f32x4)(0.0f);
+    auto fold = [&]() {
+#pragma unroll
+        for (int j = 0; j < kGemmTiles; j++)
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) tot[j][rt][v] += acc[j][rt][v];
+                acc[j][rt] = (f32x4)(0.0f);
+            }
+    };
 
     // prefetched preparation inputs
     float4 px[RPT], ps[2], pn = make_float4(1.f, 1.f, 1.f, 1.f);
@@ -1215,7 +1233,9 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
     for (int c = c0; c < cend; c += 2) {
         step(c, wb0);
         step(c + 1, wb1);
+        if (FOLD && (c - c0) % kGemmFold == kGemmFold - 2) fold();
     }
+    fold();
 
     if (NG == 2 && a.y) {
         // one K split of a gate|up pair: the up waves (slot 1) hand their
@@ -1237,7 +1257,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
                     for (int v = 0; v < 4; v++) {
                         const int r_ = rt * 16 + 4 * (lane >> 4) + v;
                         s_up[r_][64 * (wave & 1) + 16 * j + (lane & 15)] =
-                            0.0f + acc[j][rt][v] * s_unscale[r_];
+                            0.0f + tot[j][rt][v] * s_unscale[r_];
                     }
         }
         __syncthreads();
@@ -1261,7 +1281,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
                     for (int v = 0; v < 4; v++) {
                         const int r_ = rt * 16 + 4 * (lane >> 4) + v;
                         const int row = row0 + r_;
-                        const float g = 0.0f + acc[j][rt][v] * s_unscale[r_];
+                        const float g = 0.0f + tot[j][rt][v] * s_unscale[r_];
                         const float o = g / (1.0f + __expf(-g)) * s_up[r_][c];
                         if (row < a.M) a.y[(size_t)row * a.ldy + col] = o;
                         am[rt][v] = fmaxf(am[rt][v], fabsf(o * nwc));
@@ -1320,7 +1340,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
             for (int v = 0; v < 4; v++) {
                 const int r_ = rt * 16 + 4 * (lane >> 4) + v;
                 const int row = row0 + r_;
-                if (row < a.M) pp[(size_t)row * a.N + col] = acc[j][rt][v] * s_unscale[r_];
+                if (row < a.M) pp[(size_t)row * a.N + col] = tot[j][rt][v] * s_unscale[r_];
             }
     }
 }
@@ -1527,13 +1547,14 @@ __global__ __launch_bounds__(256) void k_gemm_reduce4(const float* __restrict__ 
 }
 
 template <int RT, int NG>
-int launch_gemm(const GemmArgs& a, dim3 grid) {
+int launch_gemm(const GemmArgs& a, dim3 grid, bool fold) {
+    const dim3 block(64 * kGemmWaves);
     if (a.nw)
-        hipLaunchKernelGGL((k_gemm_int4<RT, NG, kProRmsNorm>), grid, dim3(64 * kGemmWaves), 0,
-                           stream(), a);
+        hipLaunchKernelGGL((k_gemm_int4<RT, NG, kProRmsNorm, false>), grid, block, 0, stream(), a);
+    else if (NG == 1 && fold)
+        hipLaunchKernelGGL((k_gemm_int4<RT, NG, kProNone, NG == 1>), grid, block, 0, stream(), a);
     else
-        hipLaunchKernelGGL((k_gemm_int4<RT, NG, kProNone>), grid, dim3(64 * kGemmWaves), 0,
-                           stream(), a);
+        hipLaunchKernelGGL((k_gemm_int4<RT, NG, kProNone, false>), grid, block, 0, stream(), a);
     return launch_check("k_gemm_int4");
 }
 
@@ -1673,18 +1694,12 @@ extern "C" int cgk_gemm_int4_supported(int M, int K, int N, int gs, int paired) 
            (!paired || (N / 2) % 128 == 0);
 }
 
-extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs,
-                             const uint8_t* w, const float* scales_t, float smax, float* y,
-                             int ldy, int pro, const float* nw, float eps, int epi,
-                             const float* stats_in, int nstat_in, float* stats_out,
-                             const float* nw_next) {
-    const int paired = epi == kEpiSwiGlu;
-    if (!cgk_gemm_int4_supported(M, K, N, gs, paired) || ldx < K || (ldx & 3) ||
-        ((uintptr_t)x & 15) || (pro == kProRmsNorm && (!nw || ((uintptr_t)nw & 15))) ||
-        ldy < (paired ? N / 2 : N) || (size_t)M * N >= (1u << 31)) {
-        cgx_set_error("gemm_int4: unsupported shape M=%d K=%d N=%d gs=%d", M, K, N, gs);
-        return -1;
-    }
+// Launch shape of the GEMM over M rows.
+struct GemmPlan {
+    int RT, colblocks, rowblocks, ksteps, ksplit;
+};
+
+static GemmPlan gemm_plan(int M, int K, int N, int paired) {
     // row tiles per block: up to 3 (48 rows) for short batches; longer ones
     // run as blocks of 2 row tiles (32 rows), which doubles the blocks that
     // share the weights and leaves fewer K splits to reduce (measured on the
@@ -1705,6 +1720,57 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
     ksplit = ksplit < 1 ? 1 : (ksplit > 16 ? 16 : ksplit);
     const int ksteps = (nchunks + ksplit - 1) / ksplit;
     ksplit = (nchunks + ksteps - 1) / ksteps;
+    return GemmPlan{RT, colblocks, rowblocks, ksteps, ksplit};
+}
+
+// Scratch of the GEMM: the row factors, then the splits' partial sums.
+static size_t gemm_row_bytes(int M) { return (((size_t)M * 8) + 255) & ~(size_t)255; }
+
+// Whether a plain product of M rows goes to the GEMM, which reads W once per
+// row block and takes three launches, or to the GEMV, which reads W once per
+// 16 rows and takes a launch for each.  Both measured (us, GEMV / GEMM):
+//   M 64     768 x 768 16.0 / 12.8   2048 x 2048 20.4 / 13.4   4096 x 4096 34 / 24
+//   M 48     2048 x 2048 15.4 / 16.5  4096 x 4096 25.4 / 20.2  11008 x 4096 58 / 28
+//   M 32     2048 x 2048 10.6 / 12.6  4096 x 4096 17.3 / 14.9  11008 x 4096 40 / 21
+//   M 17     4096 x 4096 12.7 / 13.7  4096 x 8192 16.0 / 17.3  11008 x 4096 27 / 20
+//   M 16     4096 x 8192 10.7 / 15.2  11008 x 4096 19.2 / 16.0
+extern "C" int cgk_gemm_int4_pays(int M, int K, int N, int gs) {
+    if (!cgk_gemm_int4_supported(M, K, N, gs, 0)) return 0;
+    const size_t kn = (size_t)K * N;
+    return M > 48 || (M > 24 && kn >= (size_t)1 << 24) || (M > 16 && kn >= (size_t)5 << 23);
+}
+
+// Rows of one GEMM call (its row and output offsets are 32-bit byte offsets).
+extern "C" int cgk_gemm_int4_max_rows(int K, int N) {
+    const unsigned rows = ((1u << 29) - 1) / (unsigned)(K > N ? K : N);
+    return (int)(rows > (1u << 20) ? 1u << 20 : rows);      // 32-row blocks: grid.y < 2^16
+}
+
+// 1 when the scratch of a plain GEMM of M rows is at hand: not while the
+// stream is captured (a graph must not keep a scratch address, which a later
+// call's growth frees), nor when the device has no memory for it.
+extern "C" int cgk_gemm_int4_ready(int M, int K, int N) {
+    if (cgx_is_capturing()) return 0;
+    const GemmPlan p = gemm_plan(M, K, N, 0);
+    return cgx_scratch(CGX_SLOT_WS5, gemm_row_bytes(M) +
+                                         (p.ksplit > 1 ? (size_t)p.ksplit * M * N * 4 : 0)) != nullptr;
+}
+
+extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs,
+                             const uint8_t* w, const float* scales_t, float smax, float* y,
+                             int ldy, int pro, const float* nw, float eps, int epi,
+                             const float* stats_in, int nstat_in, float* stats_out,
+                             const float* nw_next) {
+    const int paired = epi == kEpiSwiGlu;
+    if (!cgk_gemm_int4_supported(M, K, N, gs, paired) || ldx < K || (ldx & 3) ||
+        ((uintptr_t)x & 15) || (pro == kProRmsNorm && (!nw || ((uintptr_t)nw & 15))) ||
+        ldy < (paired ? N / 2 : N) || (size_t)M * N >= (1u << 31)) {
+        cgx_set_error("gemm_int4: unsupported shape M=%d K=%d N=%d gs=%d", M, K, N, gs);
+        return -1;
+    }
+    const GemmPlan p = gemm_plan(M, K, N, paired);
+    const int RT = p.RT, colblocks = p.colblocks, rowblocks = p.rowblocks;
+    const int ksteps = p.ksteps, ksplit = p.ksplit;
     // one split storing plain rows (the lm_head of a tree verify): the GEMM
     // writes y itself, and no reduction pass copies it; one split of a
     // gate|up pair (the tree verify's 256 rows): the GEMM applies SwiGLU and
@@ -1712,7 +1778,7 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
     const bool swiglu_here = ksplit == 1 && paired && g_gemm_swiglu_here;
     const bool direct = (ksplit == 1 && epi == kEpiStore && !stats_out && ldy == N) ||
                         swiglu_here;
-    const size_t row_bytes = (((size_t)M * 8) + 255) & ~(size_t)255;
+    const size_t row_bytes = gemm_row_bytes(M);
     char* ws = (char*)cgx_scratch(CGX_SLOT_WS5,
                                   row_bytes + (direct ? 0 : (size_t)ksplit * M * N * 4));
     if (!ws) return -1;
@@ -1742,14 +1808,14 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
         return -1;
     }
     dim3 grid(colblocks, rowblocks, ksplit);
+    const bool fold = pro == kProNone && epi == kEpiStore && !stats_in && !stats_out;
     int rc;
-    if (paired) {
-        rc = RT == 1 ? launch_gemm<1, 2>(a, grid) : RT == 2 ? launch_gemm<2, 2>(a, grid)
-           : RT == 3 ? launch_gemm<3, 2>(a, grid) : launch_gemm<4, 2>(a, grid);
-    } else {
-        rc = RT == 1 ? launch_gemm<1, 1>(a, grid) : RT == 2 ? launch_gemm<2, 1>(a, grid)
-           : RT == 3 ? launch_gemm<3, 1>(a, grid) : launch_gemm<4, 1>(a, grid);
-    }
+    if (paired)
+        rc = RT == 1 ? launch_gemm<1, 2>(a, grid, fold) : RT == 2 ? launch_gemm<2, 2>(a, grid, fold)
+                                                        : launch_gemm<3, 2>(a, grid, fold);
+    else
+        rc = RT == 1 ? launch_gemm<1, 1>(a, grid, fold) : RT == 2 ? launch_gemm<2, 1>(a, grid, fold)
+                                                        : launch_gemm<3, 1>(a, grid, fold);
     if (rc || direct) return rc;
     const int Nout = paired ? N / 2 : N;
     const size_t outs = (size_t)M * Nout;

@@ -247,6 +247,29 @@ cg_tensor* cg_dequantize(cg_tensor_quant* q) {
 
 /* -------------------------------------------------------------- matmul */
 
+/* y = x @ W over a layout-3 weight: the GEMM where its rows pay for it, in
+ * calls of at most its row limit, else the GEMV. */
+static int matmul_mfma(const float* x, int M, const cg_tensor_quant* w, const cgx_qinfo* info,
+                       float* y) {
+    const int K = info->K, N = info->N, gs = info->group_size;
+    const int most = cgk_gemm_int4_max_rows(K, N);
+    for (int m0 = 0; m0 < M;) {
+        const int rows = M - m0 < most ? M - m0 : most;
+        const float* xr = x + (size_t)m0 * K;
+        float* yr = y + (size_t)m0 * N;
+        int rc;
+        if (cgk_gemm_int4_pays(rows, K, N, gs) && cgk_gemm_int4_ready(rows, K, N))
+            rc = cgk_gemm_int4(xr, K, rows, K, N, gs, w->data, w->scales, info->smax, yr, N, 0,
+                               NULL, 0.0f, 0, NULL, 0, NULL, NULL);
+        else
+            rc = cgk_gemv_mfma(xr, K, rows, K, N, gs, w->data, w->scales, yr, N, 0, NULL, 0.0f,
+                               0);
+        if (rc) return rc;
+        m0 += rows;
+    }
+    return 0;
+}
+
 int cgx_matmul_int4_dev_kernel(const float* x, int M, cg_tensor_quant* w,
                                float* y, int kernel) {
     cgx_qinfo info;
@@ -259,8 +282,8 @@ int cgx_matmul_int4_dev_kernel(const float* x, int M, cg_tensor_quant* w,
                       "(use cgx_quant_to_device)");
         return -1;
     }
-    if (kernel == 0)
-        kernel = info.layout == CGX_LAYOUT_TILED ? 1 : info.layout == CGX_LAYOUT_MFMA ? 3 : 2;
+    if (kernel == 0 && info.layout == CGX_LAYOUT_MFMA) return matmul_mfma(x, M, w, &info, y);
+    if (kernel == 0) kernel = info.layout == CGX_LAYOUT_TILED ? 1 : 2;
     if (kernel == 3 || kernel == 4) {
         if (info.layout != CGX_LAYOUT_MFMA) {
             cgx_set_error("cgx_matmul_int4: MFMA kernels need a layout-3 weight");

@@ -170,10 +170,14 @@ extern "C" int cgx_memcpy_d2d(void* dst, const void* src, size_t bytes) {
 // would record a memset node or allocate, free or synchronise then refuse:
 // memset nodes have given wrong results on replays after the first, and an
 // allocation or a synchronisation ends the capture with an error.
-static bool capturing(const char* who) {
+extern "C" int cgx_is_capturing(void) {
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(g_rt.stream, &st) != hipSuccess || st == hipStreamCaptureStatusNone)
-        return false;
+    return hipStreamIsCapturing(g_rt.stream, &st) == hipSuccess &&
+           st != hipStreamCaptureStatusNone;
+}
+
+static bool capturing(const char* who) {
+    if (!cgx_is_capturing()) return false;
     cgx_set_error("%s: the library stream is being captured into a graph (cgx_graph_begin); "
                   "only calls that allocate, clear and synchronise nothing may be captured",
                   who);

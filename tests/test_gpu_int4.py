@@ -106,6 +106,74 @@ def test_gemm_mfma_vs_oracle(gpu, oracle, rng, K, N, gs, M):
     _gemv_case(gpu, oracle, rng, K, N, gs, M, 3, 4)
 
 
+@pytest.mark.parametrize("K,N,gs,M", [(256, 128, 128, 48), (256, 128, 128, 49),
+                                      (768, 3072, 128, 97), (4096, 4096, 128, 24),
+                                      (4096, 4096, 128, 25), (11008, 4096, 128, 16),
+                                      (11008, 4096, 128, 17), (1024, 640, 128, 65),
+                                      (512, 768, 256, 50), (512, 704, 64, 70)])
+def test_matmul_dispatch_by_rows(gpu, oracle, rng, K, N, gs, M):
+    # either side of the lines between the GEMV and the GEMM, odd row counts,
+    # an odd number of 128-column slots, a group that the GEMM does not take
+    _gemv_case(gpu, oracle, rng, K, N, gs, M, 3, 0)
+
+
+def test_matmul_many_rows_wide_dynamic_range(gpu, oracle, rng):
+    # rows of very different magnitudes, a zero row and values spanning many
+    # binades through the default dispatch (the GEMM's per-row scaling)
+    K, N, gs, M = 1024, 512, 128, 64
+    data, scales = _make_weight(oracle, rng, K, N, gs)
+    scales = scales.copy()
+    scales[::7] *= 1e4
+    scales[3::11] *= 1e-6
+    x = (rng.normal(0, 1, (M, K)) * np.exp(rng.uniform(-20, 20, (M, K)))).astype(np.float32)
+    x *= np.exp(rng.uniform(-30, 30, (M, 1))).astype(np.float32)
+    x[2] = 0.0
+    y_ref = oracle_matmul(oracle, x, data, scales, K, N, gs)
+    hq, keep = host_quant_from_arrays(data, scales, K, N, gs)
+    dq = gpu.cgx_quant_to_device_layout(C.byref(hq), 3)
+    dx = DeviceArray.from_numpy(gpu, x)
+    dy = DeviceArray(gpu, M * N * 4)
+    assert gpu.cgx_matmul_int4_dev(dx.ptr, M, dq, dy.ptr) == 0, last_error(gpu)
+    assert gpu.cgx_synchronize() == 0
+    y = dy.numpy(np.float32, (M, N))
+    assert np.all(y[2] == 0.0)
+    rows = [i for i in range(M) if i != 2]
+    assert rel_err_rows(y[rows], y_ref[rows]) <= TOL
+    gpu.cg_tensor_quant_free(dq)
+
+
+def test_matmul_many_rows_under_capture(gpu, rng):
+    # a captured product takes the path without scratch memory: every replay
+    # on new inputs equals the eager GEMV, with larger eager products (which
+    # grow the scratch) between the replays
+    K, N, gs, M = 512, 256, 128, 64
+    data = rng.integers(0, 256, K * N // 2, dtype=np.uint8)
+    scales = rng.uniform(0.005, 0.02, K * N // gs).astype(np.float32)
+    hq, keep = host_quant_from_arrays(data, scales, K, N, gs)
+    dq = gpu.cgx_quant_to_device_layout(C.byref(hq), 3)
+    dx, dy = DeviceArray(gpu, M * K * 4), DeviceArray(gpu, M * N * 4)
+    de = DeviceArray(gpu, M * N * 4)
+    assert gpu.cgx_graph_begin() == 0, last_error(gpu)
+    rc = gpu.cgx_matmul_int4_dev(dx.ptr, M, dq, dy.ptr)
+    g = gpu.cgx_graph_end()
+    assert rc == 0 and g, last_error(gpu)
+    for rep in range(3):
+        x = rng.normal(0, 1, (M, K)).astype(np.float32)
+        dx.upload(x)
+        assert gpu.cgx_graph_launch(g) == 0 and gpu.cgx_synchronize() == 0, last_error(gpu)
+        y = dy.numpy(np.float32, (M, N))
+        assert gpu.cgx_matmul_int4_dev_kernel(dx.ptr, M, dq, de.ptr, 3) == 0, last_error(gpu)
+        assert gpu.cgx_synchronize() == 0
+        assert np.array_equal(y, de.numpy(np.float32, (M, N)))
+        big = 128 * (rep + 2)
+        bx, by = DeviceArray(gpu, big * K * 4), DeviceArray(gpu, big * N * 4)
+        gpu.cgx_memset(bx.ptr, 0, big * K * 4)
+        assert gpu.cgx_matmul_int4_dev(bx.ptr, big, dq, by.ptr) == 0, last_error(gpu)
+        assert gpu.cgx_synchronize() == 0
+    assert gpu.cgx_graph_free(g) == 0
+    gpu.cg_tensor_quant_free(dq)
+
+
 def _stream_case(gpu, oracle, rng, K, N, gs, M, min_units):
     """The persistent streaming GEMV (taken at K = 4096, up to 5 rows, once
     the output has min_units 32-column units per CU) against the oracle, and
