@@ -82,6 +82,41 @@ __global__ void k_kv_append(const float* __restrict__ k, const float* __restrict
     }
 }
 
+// The same for groups of 8 gt values, gt a power of two up to 64, and 16-byte
+// aligned rows: gt neighbouring lanes hold a group, 8 values each (blockIdx.y:
+// K or V), and reduce its absmax by exchanges, so that loads and stores are
+// contiguous over the wave.  Bound by memory; a thread per group, above,
+// reads 512 bytes apart from its neighbours (512 tokens of 8 heads of 128:
+// 48 -> 4 us).
+__global__ __launch_bounds__(256) void k_kv_append8(const float* __restrict__ k,
+                                                    const float* __restrict__ v, unsigned n8,
+                                                    int gt, size_t pos8, uint32_t* __restrict__ kc,
+                                                    uint32_t* __restrict__ vc,
+                                                    float* __restrict__ ks,
+                                                    float* __restrict__ vs) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;      // 8-value unit of the new rows
+    if (i >= n8) return;                                    // whole groups
+    const float* x = blockIdx.y ? v : k;
+    const float4 a = ((const float4*)x)[2 * (size_t)i], b = ((const float4*)x)[2 * (size_t)i + 1];
+    const float e[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(e[j]));
+    for (int o = 1; o < gt; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+    float s = __fdiv_rn(m, 7.0f);
+    if (s < 1e-8f) s = 1.0f;
+    uint32_t w = 0;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        int q = (int)roundf(__fdiv_rn(e[j], s));
+        q = q > 7 ? 7 : (q < -8 ? -8 : q);
+        w |= (uint32_t)(q & 0xF) << (4 * j);
+    }
+    const size_t u = pos8 + i;
+    (blockIdx.y ? vc : kc)[u] = w;
+    if ((i & (unsigned)(gt - 1)) == 0) (blockIdx.y ? vs : ks)[u / (unsigned)gt] = s;
+}
+
 // One thread per packed byte of [len][H][D/2]: (float)v * scale.
 __global__ void k_kv_get(const uint8_t* __restrict__ kc, const uint8_t* __restrict__ vc,
                          const float* __restrict__ ks, const float* __restrict__ vs,
@@ -99,6 +134,23 @@ __global__ void k_kv_get(const uint8_t* __restrict__ kc, const uint8_t* __restri
     ko[th * D + d + 1] = (float)sext4(kb >> 4) * sk;
     vo[th * D + d] = (float)sext4(vb) * sv;
     vo[th * D + d + 1] = (float)sext4(vb >> 4) * sv;
+}
+
+// The same for groups of 4 gt values and aligned rows: 4 values a thread
+// (blockIdx.y: K or V), so that a wave's stores are contiguous.
+__global__ __launch_bounds__(256) void k_kv_get4(const uint16_t* __restrict__ kc,
+                                                 const uint16_t* __restrict__ vc,
+                                                 const float* __restrict__ ks,
+                                                 const float* __restrict__ vs, unsigned n4, int gt,
+                                                 float* __restrict__ ko, float* __restrict__ vo) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const uint32_t w = (blockIdx.y ? vc : kc)[i];
+    const float s = (blockIdx.y ? vs : ks)[i / (unsigned)gt];
+    float e[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) e[j] = (float)((int)(w << (28 - 4 * j)) >> 28) * s;
+    ((float4*)(blockIdx.y ? vo : ko))[i] = make_float4(e[0], e[1], e[2], e[3]);
 }
 
 // ------------------------------------------------------------ attention
@@ -469,6 +521,17 @@ extern "C" int cgk_kv_append(const float* k, const float* v, int T, int H, int D
                              int pos, uint8_t* kc, uint8_t* vc, float* ks, float* vs) {
     int n = T * H * (D / gs);
     if (n <= 0) return 0;
+    const size_t n8 = (size_t)T * H * D / 8;
+    // whole units a group, at most a wave of lanes a group and a power of two
+    // of them, 16-byte aligned values, 4-byte aligned bytes
+    const int lanes = gs / 8;
+    if (gs % 8 == 0 && lanes <= 64 && (lanes & (lanes - 1)) == 0 && n8 <= 0xffffff00u &&
+        !(((uintptr_t)k | (uintptr_t)v) & 15) && !(((uintptr_t)kc | (uintptr_t)vc) & 3)) {
+        hipLaunchKernelGGL(k_kv_append8, dim3((unsigned)((n8 + 255) / 256), 2), dim3(256), 0,
+                           stream(), k, v, (unsigned)n8, lanes, (size_t)pos * H * D / 8,
+                           (uint32_t*)kc, (uint32_t*)vc, ks, vs);
+        return launch_check("k_kv_append8");
+    }
     hipLaunchKernelGGL(k_kv_append, dim3((n + 127) / 128), dim3(128), 0, stream(), k, v, T, H,
                        D, gs, pos, kc, vc, ks, vs);
     return launch_check("k_kv_append");
@@ -479,6 +542,14 @@ extern "C" int cgk_kv_get(const uint8_t* kc, const uint8_t* vc, const float* ks,
                           float* vo) {
     size_t nb = (size_t)len * H * (D / 2);
     if (!nb) return 0;
+    const size_t n4 = nb / 2;
+    if (gs % 4 == 0 && n4 <= 0xffffff00u && !(((uintptr_t)ko | (uintptr_t)vo) & 15) &&
+        !(((uintptr_t)kc | (uintptr_t)vc) & 1)) {
+        hipLaunchKernelGGL(k_kv_get4, dim3((unsigned)((n4 + 255) / 256), 2), dim3(256), 0,
+                           stream(), (const uint16_t*)kc, (const uint16_t*)vc, ks, vs,
+                           (unsigned)n4, gs / 4, ko, vo);
+        return launch_check("k_kv_get4");
+    }
     hipLaunchKernelGGL(k_kv_get, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, stream(),
                        kc, vc, ks, vs, len, H, D, gs, ko, vo);
     return launch_check("k_kv_get");

@@ -15,7 +15,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from cogito_amd.capi import CgFlashAttnParams, DeviceArray, last_error
+from cogito_amd.capi import CgFlashAttnParams, CgTensor, DeviceArray, last_error
 from gpu_util import host_tensor, rel_err_rows
 from oracle_lib import ptr
 from test_attn_oracle import attn_inputs, oracle_kv_fill, oracle_kv_get, orc_attention
@@ -116,6 +116,55 @@ def test_kv_write_block_and_device_get(gpu, oracle, rng):
     assert not cache_arrays(gpu, c, 0)[0].any()
     dk.free()
     dv.free()
+    gpu.cg_kv_cache_int4_free(c)
+
+
+@pytest.mark.parametrize("H,D,gs,T,pos,off", [(1, 8, 8, 1, 0, 0), (3, 64, 16, 33, 5, 0),
+                                              (2, 128, 64, 129, 1, 0), (12, 64, 64, 70, 3, 0),
+                                              (2, 48, 24, 17, 2, 0), (2, 12, 4, 9, 1, 0),
+                                              (1, 512, 512, 5, 2, 0), (8, 128, 128, 64, 7, 1)])
+def test_kv_write_get_forms(gpu, oracle, rng, H, D, gs, T, pos, off):
+    # groups of one lane to a whole wave, of a count of lanes that is no power
+    # of two, of less than a unit; rows off the 16-byte line (`off` floats);
+    # ragged lengths; zeros, infinities and values at the rounding's halves
+    S = pos + T
+    k = rng.normal(0, 1, (S, H, D)).astype(np.float32)
+    v = rng.normal(0, 2, (S, H, D)).astype(np.float32)
+    k[0, 0] = 0.0
+    v[S - 1, H - 1, :gs] = 0.0
+    k[S - 1, H - 1, :4] = [7.0, -3.5, 2.5, -0.5]
+    c = gpu.cg_kv_cache_int4_new(2, S + 1, H, D, gs)
+    assert c, last_error(gpu)
+    for lo, hi in ((0, pos), (pos, S)):
+        n = (hi - lo) * H * D
+        if not n:
+            continue
+        dk, dv = DeviceArray(gpu, n * 4 + 16), DeviceArray(gpu, n * 4 + 16)
+        for d, x in ((dk, k), (dv, v)):
+            flat = np.zeros(n + off, np.float32)
+            flat[off:] = x[lo:hi].ravel()
+            d.upload(flat)
+        assert gpu.cgx_kv_cache_int4_write(c, 1, lo, dk.ptr + 4 * off, dv.ptr + 4 * off,
+                                           hi - lo) == 0, last_error(gpu)
+    assert gpu.cgx_kv_cache_int4_set_len(c, S) == 0
+    exp = oracle_kv_fill(oracle, k, v, H, D, gs, S + 1)
+    for e, g in zip(exp, cache_arrays(gpu, c, 1)):
+        np.testing.assert_array_equal(e.view(np.uint8), g.view(np.uint8))
+    ko, vo = oracle_kv_get(oracle, *exp, S, H, D, gs)
+    n = S * H * D
+    outs = [DeviceArray(gpu, n * 4 + 16) for _ in range(2)]
+    ts = []
+    for o in outs:
+        t = CgTensor()
+        t.data = C.cast(o.ptr + 4 * off, C.POINTER(C.c_float))
+        t.ndim, t.size = 1, n
+        t.shape[0] = n
+        ts.append(t)
+    gpu.cg_kv_cache_int4_get(c, 1, C.byref(ts[0]), C.byref(ts[1]))
+    assert last_error(gpu) in ("", None), last_error(gpu)
+    for o, e in zip(outs, (ko, vo)):
+        np.testing.assert_array_equal(_bits(o.numpy(np.float32, (n + off,))[off:]),
+                                      _bits(e.ravel()))
     gpu.cg_kv_cache_int4_free(c)
 
 
