@@ -230,6 +230,21 @@ int cgk_attn_dec_batch(const float* Q, const uint8_t* kc, const uint8_t* vc, con
                        int mask_kind, const unsigned long long* anc, int tw, float* O,
                        float* stats);
 
+/* fp32 flash attention of many query rows (attn_prompt.hip), K and V packed
+ * once per call into MFMA operands.  pays: whether the call's size repays the
+ * packing.  f32 returns 0, -1 on an error, or 1 when the call has to take the
+ * fp32 kernel; afterwards *flag holds *gen when an input was not finite, and
+ * the fp32 kernel then has to run over the same output. */
+int cgk_attn_prompt_pays(int B, int Nq, int Nk, int H, int Hk, int D);
+int cgk_attn_prompt_f32(const float* Q, const float* K, const float* V, int B, int Nq, int Nk,
+                        int H, int Hk, int D, float scale, int mask_kind, int window,
+                        const float* mask, float* O, float* lse, const unsigned** flag,
+                        unsigned* gen);
+/* Merge of key splits: part_o [splits][nrow][D] and part_ml [splits][nrow][2]
+ * (maximum, sum) into O, and lse where given. */
+int cgk_attn_combine(const float* part_o, const float* part_ml, int splits, int nrow, int D,
+                     int Nq, int H, float* O, float* lse);
+
 /* Rows of a tree forward (cgx_model_forward_tree): row i sits at cache slot
  * len + i and rotary position len + rel[i]; the last tw cached keys are the
  * tree's nodes, visible to row i through anc[i]. */

@@ -306,6 +306,11 @@ int cgx_gemm_reduce4_min_blocks(int blocks);
  * the separate reduction pass (the same outputs, bit for bit); returns the
  * previous setting (-1 only reads it). */
 int cgx_gemm_swiglu_here(int on);
+/* Test hook, no reference counterpart: the flash forward takes the packed
+ * fp16 hi + lo path (head_dim 33 .. 128) from this many millions of batch *
+ * KV heads * rows * keys * head_dim (default 150; 0 always); returns the
+ * previous value (-1 only reads it). */
+int cgx_flash_packed_min(int mega);
 int cgx_attention_int4_kv_batch_dev(const float* Q, int B, int Nq, int H,
                                     cg_kv_cache_int4* cache, int slot0, const int* nk,
                                     int mask_kind, const unsigned long long* anc, int tw,

@@ -437,6 +437,79 @@ def test_flash_forward(gpu, oracle, rng, B, Nq, Nk, H, Hk, D, mt):
     assert np.all(lse[~fin] == else_[~fin])
 
 
+@pytest.fixture()
+def packed_always(gpu):
+    old = gpu.cgx_flash_packed_min(0)
+    yield
+    gpu.cgx_flash_packed_min(old)
+
+
+@pytest.mark.parametrize("B,Nq,Nk,H,Hk,D,mt,W", [
+    (1, 1, 1, 1, 1, 40, 0, 0), (1, 5, 33, 3, 2, 64, 0, 0), (2, 70, 70, 4, 2, 128, 1, 0),
+    (1, 130, 64, 2, 1, 96, 2, 9), (1, 65, 300, 6, 2, 100, 0, 0), (1, 33, 1000, 1, 1, 128, 0, 0),
+    (1, 33, 1000, 2, 1, 64, 1, 0), (1, 17, 97, 2, 2, 72, 3, 0), (3, 64, 64, 8, 8, 48, 1, 0),
+    (1, 40, 50, 5, 3, 64, 1, 0), (1, 300, 300, 2, 2, 64, 2, 40), (1, 12, 700, 2, 2, 128, 2, 5),
+    (2, 1024, 40, 32, 32, 64, 0, 0), (1, 129, 129, 4, 1, 127, 1, 0)])
+def test_flash_packed_vs_oracle(gpu, oracle, rng, packed_always, B, Nq, Nk, H, Hk, D, mt, W):
+    # one row and one key to several blocks, splits and 128-row blocks; tiles
+    # past the last key, head_dims inside a 32-dim chunk, KV heads of unequal
+    # groups, windows that leave rows without a key
+    Q, K, V = attn_inputs(rng, B, Nq, Nk, H, Hk, D)
+    mask = None
+    if mt == 3:
+        mask = rng.normal(0, 2, (Nq, Nk)).astype(np.float32)
+        mask[1, :40] = -np.inf
+        mask[2, 3:] = -FLT_MAX
+        mask[3, :] = -FLT_MAX
+    O, lse, p = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, mt, W, mask)
+    eO, else_ = orc_attention(oracle, Q, K, V, H, Hk, p.scale, mt, W, mask)
+    assert rel_err_rows(O.reshape(-1, D), eO.reshape(-1, D)) <= TOL
+    fin = else_ > -1e30
+    np.testing.assert_allclose(lse[fin], else_[fin], rtol=1e-4, atol=1e-4)
+    assert np.all(lse[~fin] == else_[~fin])
+
+
+def test_flash_packed_magnitudes(gpu, oracle, rng, packed_always):
+    # rows of Q, K and V many binades apart (the products in fp32's range):
+    # every row keeps its own scale
+    Q, K, V = attn_inputs(rng, 1, 40, 90, 4, 2, 64)
+    e = lambda n, h: np.exp2(rng.integers(-40, 40, (1, n, h, 1))).astype(np.float32)
+    ek = e(90, 2)
+    K, V = K * ek, V * e(90, 2)
+    Q = Q * np.exp2(-40).astype(np.float32)
+    Q[:, 7] = 0.0
+    V[:, 5] = 0.0
+    V[:, 6] *= np.float32(1e-38)
+    O, lse, p = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, 1, 0, None)
+    eO, _ = orc_attention(oracle, Q, K, V, 4, 2, p.scale, 1, 0, None)
+    assert rel_err_rows(O.reshape(-1, 64), eO.reshape(-1, 64)) <= TOL
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v"])
+def test_flash_packed_non_finite_inputs(gpu, rng, where):
+    # infinities and NaN give what the fp32 kernel gives, bit for bit, and
+    # leave the next call alone
+    Q, K, V = attn_inputs(rng, 1, 37, 53, 4, 2, 64)
+    fine = [x.copy() for x in (Q, K, V)]
+    x = {"q": Q, "k": K, "v": V}[where]
+    x[0, 3, 1, 5] = -np.inf
+    x[0, 9, 0, 7] = np.inf
+    x[0, 20, 1, 0] = np.nan
+    old = gpu.cgx_flash_packed_min(1 << 30)
+    try:
+        eO, el, _ = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, 1, 0, None)
+        gpu.cgx_flash_packed_min(0)
+        a, al, _ = run_flash(gpu, "cg_flash_attention_forward", *fine, 1, 0, None)
+        O, l, _ = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, 1, 0, None)
+        b, bl, _ = run_flash(gpu, "cg_flash_attention_forward", *fine, 1, 0, None)
+    finally:
+        gpu.cgx_flash_packed_min(old)
+    np.testing.assert_array_equal(O, eO)
+    np.testing.assert_array_equal(l, el)
+    np.testing.assert_array_equal(_bits(a), _bits(b))
+    np.testing.assert_array_equal(_bits(al), _bits(bl))
+
+
 def test_flash_forward_device_pointers(gpu, oracle, rng):
     B, Nq, Nk, H, Hk, D = 1, 50, 50, 4, 2, 64
     Q, K, V = attn_inputs(rng, B, Nq, Nk, H, Hk, D)
