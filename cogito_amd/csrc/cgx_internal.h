@@ -189,6 +189,13 @@ int cgk_filter_rows_ex(const float* z, int rows, int V, int top_k, float top_p,
 int cgk_filter_rows_t(const float* x, float T, float* zbuf, int rows, int V, int top_k,
                       float top_p, const float* u, int u_stride, int* tokens, int tok_every,
                       float* dist);
+/* The same over na rows of x (whose rows draw the tokens) and nb rows of x2 in
+ * the same launches; dist and zbuf hold na + nb rows.  fit: whether the scratch
+ * for so many rows is to be had. */
+int cgk_filter_rows_2(const float* x, int na, const float* x2, int nb, float T, float* zbuf,
+                      int V, int top_k, float top_p, const float* u, int u_stride, int* tokens,
+                      int tok_every, float* dist);
+int cgk_filter_rows_fit(int rows, int V, int top_k);
 
 /* ---------------------------------------- KV cache, attention, RoPE */
 /* attention mask kinds of cgk_attention */

@@ -122,6 +122,16 @@ __device__ __forceinline__ int4 block_sum_int4(int4 v, int4* lds) {
 
 // ---------------------------------------------------------------- top-p
 
+// Rows from up to two arrays: rows [0, na) at a, the ones after at b.
+struct RowsIn {
+    const float* a;
+    int na;
+    const float* b;
+    __device__ __forceinline__ const float* row(int r, int V) const {
+        return r < na ? a + (size_t)r * V : b + (size_t)(r - na) * V;
+    }
+};
+
 // z / T, elementwise (the filtered distribution's first step).
 __global__ void k_scale(const float* __restrict__ x, float* __restrict__ z, size_t n, float T) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -131,11 +141,11 @@ __global__ void k_scale(const float* __restrict__ x, float* __restrict__ z, size
 // Softmax at T = 1 of each row of z = x / T (speculative.c:81-90): max,
 // expf(z - max), running fp32 sum, division.  The rows of x are divided by T
 // as they are read (k_scale's operation, so z is never stored).
-__global__ __launch_bounds__(kThreads) void k_probs_rows(const float* __restrict__ x, int V,
-                                                         float T, float* __restrict__ probs) {
+__global__ __launch_bounds__(kThreads) void k_probs_rows(RowsIn in, int V, float T,
+                                                         float* __restrict__ probs) {
     __shared__ EosLds lds;
     EosShared& sh = lds.sh;
-    ScaledSrc src{x + (size_t)blockIdx.x * V, T};
+    ScaledSrc src{in.row(blockIdx.x, V), T};
     float* pr = probs + (size_t)blockIdx.x * V;
     if (V <= kRound) {
         // one round: the row and its exponentials stay in registers; the
@@ -224,14 +234,14 @@ __device__ __forceinline__ int certified_prefix(const float (&x)[kCh], int V, fl
 }
 
 // Cutoff, draw and the filtered distribution of top-p over one row: `probs`
-// (index order) and `sorted` (descending).  Rows r with (r + 1) % tok_every
-// == 0 draw a token (tokens[r / tok_every], draw u[(r / tok_every) *
+// (index order) and `sorted` (descending).  Rows r < tok_rows with (r + 1) %
+// tok_every == 0 draw a token (tokens[r / tok_every], draw u[(r / tok_every) *
 // u_stride]; tok_every 0: none); every row writes its distribution when
 // dist is given.  ws holds 2V ints per row.
 __global__ __launch_bounds__(kThreads) void k_top_p_finish(
     const float* __restrict__ probs, const float* __restrict__ sorted, int V, float top_p,
     const float* __restrict__ u, int u_stride, int* __restrict__ tokens, int tok_every,
-    float* __restrict__ dist, int* __restrict__ ws) {
+    int tok_rows, float* __restrict__ dist, int* __restrict__ ws) {
     __shared__ EosShared sh;
     __shared__ int lds[kWaves];
     __shared__ int4 lds4[kWaves];
@@ -278,7 +288,7 @@ __global__ __launch_bounds__(kThreads) void k_top_p_finish(
     // (every element >= vc kept, right unless the tie group of vc is cut),
     // finds the element holding the token's value and counts the elements
     // above and equal to both values.
-    const bool want_tok = tokens && tok_every > 0 && (row + 1) % tok_every == 0;
+    const bool want_tok = tokens && tok_every > 0 && row < tok_rows && (row + 1) % tok_every == 0;
     const int ti = want_tok ? row / tok_every : 0;
     int pos = 0;
     if (want_tok) {
@@ -379,11 +389,11 @@ __device__ __forceinline__ unsigned long long topk_entry(uint32_t key, int j) {
 // Top-k over one row of z (k < V, k <= kTopKMax), then either a token
 // (cg_sample_top_k; with top_p < 1 the nucleus rule over the list) or the
 // filtered distribution (dense row).
-__global__ __launch_bounds__(kThreads) void k_top_k(const float* __restrict__ z, int V, int k,
+__global__ __launch_bounds__(kThreads) void k_top_k(RowsIn z, int V, int k,
                                                     int kpow2, float top_p,
                                                     const float* __restrict__ u, int u_stride,
                                                     int* __restrict__ tokens, int tok_every,
-                                                    float* __restrict__ dist,
+                                                    int tok_rows, float* __restrict__ dist,
                                                     int* __restrict__ lidx,
                                                     float* __restrict__ lp,
                                                     const unsigned long long* __restrict__ gcand,
@@ -397,7 +407,7 @@ __global__ __launch_bounds__(kThreads) void k_top_k(const float* __restrict__ z,
     __shared__ int lds[kWaves];
     __shared__ int s_digit, s_need, s_ncand;
     const int row = blockIdx.x, t = threadIdx.x, wv = t >> 6;
-    const float* zr = z + (size_t)row * V;
+    const float* zr = z.row(row, V);
     const uint32_t kfloor = order_key(kTopKFloor);
 
     // The row is read in coalesced sweeps of kU values per thread, whose loads
@@ -563,7 +573,7 @@ __global__ __launch_bounds__(kThreads) void k_top_k(const float* __restrict__ z,
     RowSrc vs{vals};
     // this row's token (rows r with (r + 1) % tok_every == 0): tokens[ti]
     // with the draw u[ti * u_stride]
-    const bool want_tok = tokens && tok_every > 0 && (row + 1) % tok_every == 0;
+    const bool want_tok = tokens && tok_every > 0 && row < tok_rows && (row + 1) % tok_every == 0;
     const int ti = want_tok ? row / tok_every : 0;
     const bool more = dist || lidx;      // a distribution or list after the token
     if (want_tok && !use_p) {
@@ -634,13 +644,13 @@ __global__ void k_topk_zero(int* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0;
 }
 
-__global__ __launch_bounds__(kTKThreads) void k_topk_hist(const float* __restrict__ z, int V,
+__global__ __launch_bounds__(kTKThreads) void k_topk_hist(RowsIn z, int V,
                                                          int* __restrict__ hist) {
     __shared__ int h[kHBins];
     const int row = blockIdx.y, tile = blockIdx.x, t = threadIdx.x;
     for (int i = t; i < kHBins; i += kTKThreads) h[i] = 0;
     __syncthreads();
-    const float* zr = z + (size_t)row * V + (size_t)tile * kTK;
+    const float* zr = z.row(row, V) + (size_t)tile * kTK;
     const int n = min(kTK, V - tile * kTK);
     float xs[kTK / kTKThreads];
 #pragma unroll
@@ -657,7 +667,7 @@ __global__ __launch_bounds__(kTKThreads) void k_topk_hist(const float* __restric
         if (h[i]) atomicAdd(&gh[i], h[i]);
 }
 
-__global__ __launch_bounds__(kTKThreads) void k_topk_collect(const float* __restrict__ z, int V,
+__global__ __launch_bounds__(kTKThreads) void k_topk_collect(RowsIn z, int V,
                                                             int k, const int* __restrict__ hist,
                                                             int* __restrict__ state,
                                                             unsigned long long* __restrict__ gcand) {
@@ -708,7 +718,7 @@ __global__ __launch_bounds__(kTKThreads) void k_topk_collect(const float* __rest
         return;
     }
     const uint32_t bin = (uint32_t)s_bin;
-    const float* zr = z + (size_t)row * V + (size_t)tile * kTK;
+    const float* zr = z.row(row, V) + (size_t)tile * kTK;
     const int n = min(kTK, V - tile * kTK);
 #pragma unroll
     for (int q = 0; q < kTK / kTKThreads; q++) {
@@ -723,14 +733,20 @@ __global__ __launch_bounds__(kTKThreads) void k_topk_collect(const float* __rest
     }
 }
 
+// Scratch of the candidate pass over `rows` rows.
+size_t topk_bytes(int rows) {
+    return (size_t)rows * ((kHBins + kTKState) * 4 + kTopKMax * 8) + 256;
+}
+
 // Launch of k_top_k, through the multi-workgroup candidate pass for long rows.
-int launch_top_k(const float* z, int rows, int V, int k, int kpow2, float top_p, const float* u,
-                 int u_stride, int* tokens, int tok_every, float* dist, int* lidx, float* lp) {
+int launch_top_k(const RowsIn& z, int rows, int V, int k, int kpow2, float top_p, const float* u,
+                 int u_stride, int* tokens, int tok_every, int tok_rows, float* dist, int* lidx,
+                 float* lp) {
     const unsigned long long* gcand = nullptr;
     const int* gstate = nullptr;
     if (V >= 4 * kTK) {
         const size_t hn = (size_t)rows * (kHBins + kTKState);
-        char* w = (char*)cgx_scratch(CGX_SLOT_WS6, hn * 4 + (size_t)rows * kTopKMax * 8 + 256);
+        char* w = (char*)cgx_scratch(CGX_SLOT_WS6, topk_bytes(rows));
         if (!w) return -1;
         int* hist = (int*)w;
         int* state = hist + (size_t)rows * kHBins;
@@ -747,7 +763,7 @@ int launch_top_k(const float* z, int rows, int V, int k, int kpow2, float top_p,
         gstate = state;
     }
     hipLaunchKernelGGL(k_top_k, dim3(rows), dim3(kThreads), 0, stream(), z, V, k, kpow2, top_p,
-                       u, u_stride, tokens, tok_every, dist, lidx, lp, gcand, gstate);
+                       u, u_stride, tokens, tok_every, tok_rows, dist, lidx, lp, gcand, gstate);
     return launch_check("k_top_k");
 }
 
@@ -888,8 +904,8 @@ extern "C" int cgk_typical_rows(const float* logits, int rows, int V, float typi
     uint32_t* skeys = (uint32_t*)(w + 4 * a);
     uint32_t* perm = (uint32_t*)(w + 5 * a);
     void* sws = w + 6 * a;
-    hipLaunchKernelGGL(k_probs_rows, dim3(rows), dim3(kThreads), 0, stream(), logits, V, 1.0f,
-                       probs);
+    hipLaunchKernelGGL(k_probs_rows, dim3(rows), dim3(kThreads), 0, stream(),
+                       RowsIn{logits, rows, nullptr}, V, 1.0f, probs);
     if (launch_check("k_probs_rows")) return -1;
     hipLaunchKernelGGL(k_typ_scores, dim3(rows), dim3(kThreads), 0, stream(), probs, V, nl, terms,
                        keys);
@@ -918,8 +934,8 @@ extern "C" int cgk_topk_lists(const float* z, int rows, int V, int top_k, float 
     }
     int kpow2 = 64;
     while (kpow2 < top_k) kpow2 <<= 1;
-    return launch_top_k(z, rows, V, top_k, kpow2, top_p, nullptr, 0, nullptr, 0, nullptr, lidx,
-                        lp);
+    return launch_top_k(RowsIn{z, rows, nullptr}, rows, V, top_k, kpow2, top_p, nullptr, 0, nullptr,
+                        0, 0, nullptr, lidx, lp);
 }
 
 extern "C" int cgk_scale(const float* x, float* z, size_t n, float T) {
@@ -945,9 +961,37 @@ extern "C" int cgk_filter_rows_ex(const float* z, int rows, int V, int top_k, fl
 extern "C" int cgk_filter_rows_t(const float* x, float T, float* zbuf, int rows, int V,
                                  int top_k, float top_p, const float* u, int u_stride,
                                  int* tokens, int tok_every, float* dist) {
+    return cgk_filter_rows_2(x, rows, nullptr, 0, T, zbuf, V, top_k, top_p, u, u_stride, tokens,
+                             tok_every, dist);
+}
+
+// Scratch of cgk_filter_rows_2's top-p path.
+static size_t top_p_bytes(int rows, int V, size_t* wsb) {
+    const size_t n = (size_t)rows * V, sb = cgk_row_sort_ws(rows, V, 0);
+    *wsb = sb > n * 8 ? sb : n * 8;
+    return n * 8 + *wsb;
+}
+
+// Whether the scratch for `rows` rows in one call is to be had.
+extern "C" int cgk_filter_rows_fit(int rows, int V, int top_k) {
+    if (rows > 65535) return 0;
+    size_t wsb;
+    void* p = top_k > 0 && top_k < V
+                  ? cgx_scratch(CGX_SLOT_WS6, topk_bytes(rows))
+                  : cgx_scratch(CGX_SLOT_WS0, top_p_bytes(rows, V, &wsb));
+    if (!p) cgx_clear_error();
+    return p != nullptr;
+}
+
+// The same over rows of two arrays at once: na rows of x (whose rows draw the
+// tokens), then nb rows of x2; dist and zbuf hold na + nb rows.
+extern "C" int cgk_filter_rows_2(const float* x, int na, const float* x2, int nb, float T,
+                                 float* zbuf, int V, int top_k, float top_p, const float* u,
+                                 int u_stride, int* tokens, int tok_every, float* dist) {
+    const int rows = na + nb;
     if (!tokens) tok_every = 0;
-    if (rows <= 0 || V <= 0 || rows > 65535 || (!tok_every && !dist) || tok_every < 0 ||
-        (tok_every && !u)) {
+    if (na <= 0 || nb < 0 || V <= 0 || rows > 65535 || (!tok_every && !dist) || tok_every < 0 ||
+        (tok_every && !u) || (nb && !x2)) {
         cgx_set_error("filter: invalid arguments");
         return -1;
     }
@@ -962,37 +1006,37 @@ extern "C" int cgk_filter_rows_t(const float* x, float T, float* zbuf, int rows,
         }
         int kpow2 = 64;
         while (kpow2 < top_k) kpow2 <<= 1;
-        const float* z = x;
+        RowsIn z{x, na, x2};
         if (T != 1.0f) {
             if (!zbuf) {
                 cgx_set_error("filter: top-k at T != 1 needs a workspace for x / T");
                 return -1;
             }
-            if (cgk_scale(x, zbuf, (size_t)rows * V, T)) return -1;
-            z = zbuf;
+            const size_t n = (size_t)na * V;
+            if (cgk_scale(x, zbuf, n, T) || cgk_scale(x2, zbuf + n, (size_t)nb * V, T)) return -1;
+            z = RowsIn{zbuf, rows, nullptr};
         }
-        return launch_top_k(z, rows, V, top_k, kpow2, top_p, u, u_stride, tokens, tok_every,
+        return launch_top_k(z, rows, V, top_k, kpow2, top_p, u, u_stride, tokens, tok_every, na,
                             dist, nullptr, nullptr);
     }
     // the descending sort of each row's probabilities (rowsort.hip, on the
     // values' bit patterns, monotone for non-negative floats) shares its
     // workspace with the finish's
-    size_t n = (size_t)rows * V;
-    size_t wsb = n * 8;
-    const size_t sb = cgk_row_sort_ws(rows, V, 0);
-    if (sb > wsb) wsb = sb;
-    char* w = (char*)cgx_scratch(CGX_SLOT_WS0, n * 8 + wsb);
+    const size_t n = (size_t)rows * V;
+    size_t wsb;
+    char* w = (char*)cgx_scratch(CGX_SLOT_WS0, top_p_bytes(rows, V, &wsb));
     if (!w) return -1;
     float* probs = (float*)w;
     float* sorted = probs + n;
     int* ws = (int*)(sorted + n);
-    hipLaunchKernelGGL(k_probs_rows, dim3(rows), dim3(kThreads), 0, stream(), x, V, T, probs);
+    hipLaunchKernelGGL(k_probs_rows, dim3(rows), dim3(kThreads), 0, stream(), RowsIn{x, na, x2}, V,
+                       T, probs);
     if (launch_check("k_probs_rows")) return -1;
     if (cgk_row_sort((const uint32_t*)probs, nullptr, rows, V, 1, (uint32_t*)sorted, nullptr, ws,
                      wsb))
         return -1;
     hipLaunchKernelGGL(k_top_p_finish, dim3(rows), dim3(kThreads), 0, stream(), probs, sorted,
-                       V, top_p, u, u_stride, tokens, tok_every, dist, ws);
+                       V, top_p, u, u_stride, tokens, tok_every, na, dist, ws);
     return launch_check("k_top_p_finish");
 }
 

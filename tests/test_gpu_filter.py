@@ -271,6 +271,39 @@ def test_filtered_verify_batch_device(gpu, oracle, rng):
         d.free()
 
 
+@pytest.mark.parametrize("B,V,gamma,T,k,p", [
+    (2, 7, 1, 1.0, 0, 0.9),                 # the fewest rows of each side
+    (2, 33000, 1, 0.8, 0, 0.9),             # rows of two scan rounds
+    (2, 33000, 3, 1.0, 50, 1.0),            # long rows' candidate pass, unscaled
+    (2, 33000, 3, 0.7, 50, 0.9),            # and scaled
+    (5, 500, 7, 1.0, 0, 0.8),
+])
+def test_filtered_verify_rows_of_both_arrays(gpu, oracle, rng, B, V, gamma, T, k, p):
+    """Target and draft rows share the filter's launches: every chain of a batch
+    gets the oracle's ratios and tokens, whichever array its rows come from."""
+    print(f"verify B={B} V={V} g={gamma} T={T} k={k} p={p}", flush=True)
+    ins = [verify_inputs(oracle, rng, V, gamma, T, k, p, b % 2 == 0) for b in range(B)]
+    arrs = [np.stack([i[j] for i in ins]) for j in range(4)]
+    devs = [DeviceArray.from_numpy(gpu, a) for a in arrs]
+    dout, dn = DeviceArray(gpu, B * (gamma + 1) * 4), DeviceArray(gpu, B * 4)
+    dap = DeviceArray(gpu, B * gamma * 4)
+    assert gpu.cgx_verify_chain_batch_dev(*(d.ptr for d in devs), B, gamma, V, T, k, p, dout.ptr,
+                                          dn.ptr, dap.ptr) == 0, last_error(gpu)
+    gpu.cgx_synchronize()
+    out, n = dout.numpy(np.int32, (B, gamma + 1)), dn.numpy(np.int32, (B,))
+    ap = dap.numpy(np.float32, (B, gamma))
+    for b in range(B):
+        o, ap_o = np.zeros(gamma + 1, np.int32), np.zeros(gamma, np.float32)
+        rows = [np.ascontiguousarray(a[b]) for a in arrs]
+        n_o = oracle.orc_verify_chain(*(ptr(r) for r in rows), gamma, V, T, k, p, ptr(o),
+                                      ptr(ap_o))
+        assert n[b] == n_o
+        np.testing.assert_array_equal(out[b, :n_o + 1], o[:n_o + 1])
+        np.testing.assert_array_equal(_bits(ap[b]), _bits(ap_o))
+    for d in (*devs, dout, dn, dap):
+        d.free()
+
+
 def test_dropin_top_k_top_p_follow_reference_lcg(gpu, oracle, rng):
     gpu.cgx_lcg_seed(42)
     mirror = LCG(42)
