@@ -366,6 +366,120 @@ __global__ void k_matmul_generic(const float* __restrict__ x, int M, int K,
     y[o] = sum;
 }
 
+// The same sums with the products taken out of their serial chains.  Only the
+// additions have to follow each other; what k_matmul_generic spends its time
+// on is everything else, in one thread per output: a 64-bit division by the
+// group size, the loads (each a wait) and two products.  Here a block of 8
+// waves owns 64 columns x R rows and walks K in steps of kRefK: every wave
+// forms the products of 8 k's (its weights and scales loaded a step ahead,
+// decoded once for the R rows) and leaves them in LDS; wave r then adds row
+// r's of the step before, column = lane, in order.  Two buffers, one barrier a
+// step.  Bound by a step's latency (a wave's 64 dependent additions, the next
+// step's loads): about 1.05 us a step at R = 1, 1.3 at R = 2, 2.2 at R = 4.
+// One row of 2400 x 4000 (groups of 32): 796 -> 49 us; 12 rows 924 -> 64;
+// one row of 4096 x 4096 (groups of 100): 1087 -> 78.
+constexpr int kRefK = 64, kRefWaves = 8, kRefPer = kRefK / kRefWaves, kRefCols = 64;
+
+// n / d for n < 2^31: mulhi(n, mul) >> sh with mul = ceil(2^(32 + sh) / d) and
+// 2^(sh + 1) >= d.  mul d - 2^(32 + sh) < d, so n times it is below 2^(32 + sh)
+// and the quotient's fraction cannot reach the next whole.  d = 1: mul 0.
+struct Div31 {
+    unsigned mul, sh;
+    __device__ __forceinline__ unsigned div(unsigned n) const {
+        return mul ? __umulhi(n, mul) >> sh : n;
+    }
+};
+
+template <int R>
+__global__ __launch_bounds__(64 * kRefWaves) void k_matmul_ref(
+    const float* __restrict__ x, int M, int K, int N, Div31 gs,
+    const uint8_t* __restrict__ data, const float* __restrict__ scales, float* __restrict__ y,
+    int colblocks, int items) {
+    __shared__ float prod[2][R][kRefK][kRefCols];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int steps = (K + kRefK - 1) / kRefK;
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int j = (item % colblocks) * kRefCols + lane, i0 = item / colblocks * R;
+        const int jc = min(j, N - 1);
+        unsigned w[kRefPer];
+        float sc[kRefPer], xv[R][kRefPer];
+        // k's past K and rows past M load the last ones; their products are
+        // not added
+        auto load = [&](int step) {
+            const int k0 = step * kRefK + wv * kRefPer;
+            auto one = [&](int q, int k) {
+                const unsigned o = (unsigned)k * (unsigned)N + (unsigned)jc;
+                w[q] = (unsigned)data[o >> 1] >> ((o & 1u) * 4u);
+                sc[q] = scales[gs.div(o)];
+            };
+            if (k0 + kRefPer <= K) {
+#pragma unroll
+                for (int q = 0; q < kRefPer; q++) one(q, k0 + q);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const float* xr = x + (size_t)min(i0 + r, M - 1) * K + k0;
+#pragma unroll
+                    for (int q = 0; q < kRefPer; q++) xv[r][q] = xr[q];
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < kRefPer; q++) one(q, min(k0 + q, K - 1));
+#pragma unroll
+                for (int r = 0; r < R; r++)
+#pragma unroll
+                    for (int q = 0; q < kRefPer; q++)
+                        xv[r][q] = x[(size_t)min(i0 + r, M - 1) * K + min(k0 + q, K - 1)];
+            }
+        };
+        auto products = [&](int buf) {
+#pragma unroll
+            for (int q = 0; q < kRefPer; q++) {
+                const float wf = (float)((int)(w[q] << 28) >> 28);
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    prod[buf][r][wv * kRefPer + q][lane] =
+                        __fmul_rn(__fmul_rn(xv[r][q], wf), sc[q]);
+            }
+        };
+        float sum = 0.0f;
+        load(0);
+        products(0);
+        load(min(1, steps - 1));
+        __syncthreads();
+        for (int t = 0; t < steps; t++) {
+            if (t + 1 < steps) {
+                products((t + 1) & 1);
+                load(min(t + 2, steps - 1));
+            }
+            if (wv < R) {
+                const float(*p)[kRefCols] = prod[t & 1][wv];
+                const int n = min(kRefK, K - t * kRefK);
+                if (n == kRefK) {
+#pragma unroll
+                    for (int q = 0; q < kRefK; q++) sum = __fadd_rn(sum, p[q][lane]);
+                } else {
+                    for (int q = 0; q < n; q++) sum = __fadd_rn(sum, p[q][lane]);
+                }
+            }
+            __syncthreads();
+        }
+        if (wv < R && i0 + wv < M && j < N) y[(size_t)(i0 + wv) * N + j] = sum;
+    }
+}
+
+template <int R>
+int launch_ref(const float* x, int M, int K, int N, Div31 gs, const uint8_t* flat,
+               const float* scales, float* y) {
+    const int colblocks = (N + kRefCols - 1) / kRefCols;
+    const size_t items = (size_t)colblocks * ((M + R - 1) / R);
+    if (items > 0x7fffffffu - 65536u) return 1;
+    hipLaunchKernelGGL(k_matmul_ref<R>, dim3((unsigned)(items < 65536 ? items : 65536)),
+                       dim3(64 * kRefWaves), 0, stream(), x, M, K, N, gs, flat, scales, y,
+                       colblocks, (int)items);
+    return launch_check("k_matmul_ref");
+}
+
 template <int M, int PRO>
 int launch_gemv_m(const float* x, int K, int N, int gs, const uint8_t* tiled,
                   const float* scales_t, float* y, const GemvEpi& ep) {
@@ -495,9 +609,28 @@ extern "C" int cgk_int4_gemv_tiled(const float* x, int M, int K, int N, int gs,
                                0);
 }
 
+// Whether a flat product goes to k_matmul_ref: from one whole step of K (2000
+// rows of 13 x 37 took 5.2 us in k_matmul_generic and 9.7 there; 300 x 30 with
+// 2000 rows 65 and 25), and element indexes of 31 bits.  Its blocks take one
+// row while the launch has no more than two blocks a CU, two rows above (2400 x
+// 4000: 8 rows 54 us with one and 55 with two, 12 rows 66 and 64, 40 rows 209
+// and 167).
+static bool ref_pays(int M, int K, int N, int gs) {
+    return M > 0 && N > 0 && gs > 0 && K >= kRefK && (long long)K * N <= 0x7fffffffll;
+}
+
 extern "C" int cgk_int4_matmul_generic(const float* x, int M, int K, int N,
                                        int gs, const uint8_t* flat,
                                        const float* scales, float* y) {
+    if (ref_pays(M, K, N, gs)) {
+        unsigned sh = 0;
+        while ((2u << sh) < (unsigned)gs) sh++;
+        const Div31 dv{gs == 1 ? 0u : (unsigned)(((1ull << (32 + sh)) + gs - 1) / gs), sh};
+        const long long blocks = (long long)((N + kRefCols - 1) / kRefCols) * M;
+        const int rc = blocks <= 512 ? launch_ref<1>(x, M, K, N, dv, flat, scales, y)
+                                     : launch_ref<2>(x, M, K, N, dv, flat, scales, y);
+        if (rc <= 0) return rc;
+    }
     size_t outs = (size_t)M * N;
     hipLaunchKernelGGL(k_matmul_generic, dim3((unsigned)((outs + 255) / 256)),
                        dim3(256), 0, stream(), x, M, K, N, gs, flat, scales, y);

@@ -286,6 +286,39 @@ def test_generic_kernel_bitexact(gpu, oracle, rng, M, K, N, gs):
     gpu.cg_tensor_free(ty)
 
 
+@pytest.mark.parametrize("M,K,N,gs", [
+    (1, 63, 65, 3),                         # below one step: thread per output
+    (1, 64, 1, 1), (2, 65, 63, 2), (3, 128, 64, 7), (5, 191, 129, 129),
+    (513, 71, 33, 40), (514, 64, 64, 10 ** 6), (9, 130, 4160, 100),
+])
+def test_reference_order_matmul_edges(gpu, oracle, rng, M, K, N, gs):
+    """Ragged steps, columns and rows, one row or two a block: bit for bit the
+    reference's sums, signed zeros, infinities and NaN among the inputs."""
+    print(f"flat M={M} K={K} N={N} gs={gs}", flush=True)
+    w = rng.normal(0, 0.02, (K, N)).astype(np.float32)
+    w.flat[0:min(gs, K * N // 2)] = 0.0     # a group of scale 0
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    x[0, 0], x[0, K - 1] = -0.0, 1e-42
+    if M > 1:
+        x[1, K // 2] = np.inf
+    if M > 2:
+        x[2, K - 1] = np.nan
+    data, scales = oracle_quantize(oracle, w, gs)
+    y_ref = oracle_matmul(oracle, x, data, scales, K, N, gs)
+    hq, keep = host_quant_from_arrays(data, scales, K, N, gs)
+    tx = host_tensor(gpu, x)
+    ty = host_tensor(gpu, np.full((M, N), 7.0, np.float32))
+    gpu.cgx_clear_error()
+    gpu.cg_matmul_int4(tx, C.byref(hq), ty)
+    assert last_error(gpu) == "", last_error(gpu)
+    y = tensor_np(gpu, ty)
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(y_ref))
+    num = ~np.isnan(y_ref)                  # a NaN's sign is not part of the contract
+    np.testing.assert_array_equal(_bits(y[num]), _bits(y_ref[num]))
+    gpu.cg_tensor_free(tx)
+    gpu.cg_tensor_free(ty)
+
+
 def test_gemv_api_host_io_device_weight(gpu, oracle, rng):
     K, N, gs = 512, 256, 128
     data, scales = _make_weight(oracle, rng, K, N, gs)
