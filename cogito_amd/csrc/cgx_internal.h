@@ -92,7 +92,7 @@ int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs, const ui
  * hand (not under stream capture). */
 int cgk_gemm_int4_pays(int M, int K, int N, int gs);
 int cgk_gemm_int4_max_rows(int K, int N);
-int cgk_gemm_int4_ready(int M, int K, int N);
+int cgk_gemm_int4_ready(int M, int K, int N, int gs);
 int cgk_absmax(const float* s, size_t n, float* out_host);
 int cgk_gemv_mfma(const float* x, int ldx, int M, int K, int N, int gs, const uint8_t* w,
                   const float* scales_t, float* y, int ldy, int pro, const float* nw, float eps,

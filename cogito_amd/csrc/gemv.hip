@@ -940,6 +940,15 @@ int launch_pe(const MfmaArgs& a, int T) {
 // multiplied.  K is split over blockIdx.z; k_gemm_reduce sums the splits in
 // a fixed order and applies the epilogue (store, accumulate, SwiGLU of the
 // gate|up pair).
+//
+// Scale groups of 64 and 32 columns (plain products) take slots of 64 and 32
+// columns, 2 and 1 tiles a wave (GT): every slot needs its own scaled copy of
+// the activations, so a product of the narrower groups spends more of its time
+// preparing and reading A.  Against the GEMV in chunks of 16 rows (us, GEMV /
+// groups of 64 / of 32): 400 x 4096 x 8192 253 / 92 / 127, 400 x 11008 x 4096
+// 440 / 125 / 182, 64 x 4096 x 4096 36 / 21 / 22, 48 x 2048 x 2048 15.8 / 13.8
+// / 13.8; their errors against 64 bits 1.5 to 2.0e-7 of the result, the GEMV's
+// 1.9 to 2.1e-7.
 
 constexpr int kGemmWaves = 4;
 constexpr int kGemmTiles = 4;            // column tiles per wave
@@ -975,8 +984,10 @@ struct GemmArgs {
     const float* nw_next;     // the next linear's RMSNorm weights, or nullptr
 };
 
-template <int RT, int NG, int PRO, bool FOLD>
+template <int RT, int NG, int PRO, bool FOLD, int GT = kGemmTiles>
 __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
+    static_assert(GT == kGemmTiles || (NG == 1 && PRO == kProNone), "pairs have 128-column slots");
+    constexpr int SW = 32 * GT;                 // slot width
     constexpr int BM = 16 * RT;
     constexpr int RPT = BM / 8;                 // rows prepared per thread
     __shared__ _Float16 sa[2][2][BM][kGemmRowH];
@@ -999,7 +1010,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
         bx = q / gy;
         by = q % gy;
     }
-    // slots: logical 128-column groups and their scale-group rows
+    // slots: logical SW-column groups and their scale-group rows
     int slot_ok[2], grp[2], lcol[2];
 #pragma unroll
     for (int s = 0; s < 2; s++) {
@@ -1007,7 +1018,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
             lcol[s] = (s ? a.ff : 0) + 128 * bx;
             slot_ok[s] = 1;
         } else {
-            lcol[s] = 128 * (2 * bx + s);
+            lcol[s] = SW * (2 * bx + s);
             slot_ok[s] = lcol[s] < a.N;
         }
         grp[s] = slot_ok[s] ? lcol[s] / a.gs : 0;
@@ -1071,8 +1082,8 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
             s_unscale[threadIdx.x] = a.unscale[min(row0 + (int)threadIdx.x, a.M - 1)];
     }
 
-    // ---- this wave's tiles: slot ws, tiles 4 (wave & 1) + j of the slot.  A
-    // wave of a missing slot (odd number of 128-column slots) runs on tile 0
+    // ---- this wave's tiles: slot ws, tiles GT (wave & 1) + j of the slot.  A
+    // wave of a missing slot (odd number of slots) runs on tile 0
     // and stores nothing, so that every wave takes the same path.
     const int ws = wave >> 1;
     const int wave_ok = slot_ok[ws];
@@ -1087,34 +1098,34 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
         (void*)a.scales_t, (short)0, (int)((size_t)(a.N / a.gs) * a.K * 4), kBufWord3);
     const __amdgpu_buffer_rsrc_t rn = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(PRO == kProRmsNorm ? a.nw : a.scales_t), (short)0, a.K * 4, kBufWord3);
-    int wo[kGemmTiles];
+    int wo[GT];
 #pragma unroll
-    for (int j = 0; j < kGemmTiles; j++) {
-        const int t = 4 * (wave & 1) + j;               // tile within the slot
-        const int L = paired ? 2 * (8 * bx + t) + ws : 8 * (2 * bx + ws) + t;
+    for (int j = 0; j < GT; j++) {
+        const int t = GT * (wave & 1) + j;              // tile within the slot
+        const int L = paired ? 2 * (8 * bx + t) + ws : 2 * GT * (2 * bx + ws) + t;
         wo[j] = (wave_ok ? L : 0) * nchunks * kChunkBytes + 16 * lane;
     }
     // steps run in pairs; a step at or past c1 (odd count) prepares zeros and
     // reads the split's last chunk again
     const int cend = c0 + ((c1 - c0 + 1) & ~1);
-    auto wload = [&](int c, u32x4 (&d)[kGemmTiles]) {
+    auto wload = [&](int c, u32x4 (&d)[GT]) {
         const int off = min(c, c1 - 1) * kChunkBytes;
 #pragma unroll
-        for (int j = 0; j < kGemmTiles; j++)
+        for (int j = 0; j < GT; j++)
             d[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, wo[j], off, 2));
     };
-    u32x4 wb0[kGemmTiles], wb1[kGemmTiles];
+    u32x4 wb0[GT], wb1[GT];
     __builtin_amdgcn_sched_barrier(0);
     wload(c0, wb0);
 
-    f32x4 acc[kGemmTiles][RT], tot[kGemmTiles][RT];
+    f32x4 acc[GT][RT], tot[GT][RT];
 #pragma unroll
-    for (int j = 0; j < kGemmTiles; j++)
+    for (int j = 0; j < GT; j++)
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) acc[j][rt] = tot[j][rt] = (f32x4)(0.0f);
     auto fold = [&]() {
 #pragma unroll
-        for (int j = 0; j < kGemmTiles; j++)
+        for (int j = 0; j < GT; j++)
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
@@ -1154,7 +1165,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
 
     // sched_barrier(0) keeps the phases in this order, so that the waits
     // for the loads of the next step fall where they are consumed
-    auto step = [&](int c, u32x4 (&wcur)[kGemmTiles]) {
+    auto step = [&](int c, u32x4 (&wcur)[GT]) {
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();                       // the previous step's A reads are done
         const float4 n4 = pn;
@@ -1207,9 +1218,9 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
         __syncthreads();
 #pragma unroll
         for (int kb = 0; kb < 4; kb++) {
-            f16x8 b[kGemmTiles];
+            f16x8 b[GT];
 #pragma unroll
-            for (int j = 0; j < kGemmTiles; j++) {
+            for (int j = 0; j < GT; j++) {
                 const uint32_t word = kb == 0 ? wcur[j].x : kb == 1 ? wcur[j].y
                                     : kb == 2 ? wcur[j].z : wcur[j].w;
                 b[j] = nib_to_f16(word, nk);
@@ -1220,7 +1231,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
                 const f16x8 ah = *(const f16x8*)&sa[ws][0][ar][ak];
                 const f16x8 al = *(const f16x8*)&sa[ws][1][ar][ak];
 #pragma unroll
-                for (int j = 0; j < kGemmTiles; j++) {
+                for (int j = 0; j < GT; j++) {
                     acc[j][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b[j], acc[j][rt], 0, 0, 0);
                     acc[j][rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b[j], acc[j][rt], 0, 0, 0);
                 }
@@ -1250,7 +1261,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
         __syncthreads();
         if (ws == 1) {
 #pragma unroll
-            for (int j = 0; j < kGemmTiles; j++)
+            for (int j = 0; j < GT; j++)
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -1271,7 +1282,7 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
                     ss[rt][v] = 0.0f;
                 }
 #pragma unroll
-            for (int j = 0; j < kGemmTiles; j++) {
+            for (int j = 0; j < GT; j++) {
                 const int c = 64 * (wave & 1) + 16 * j + (lane & 15);
                 const int col = 128 * bx + c;
                 const float nwc = a.nw_next ? a.nw_next[col] : 1.0f;
@@ -1332,8 +1343,8 @@ __global__ __launch_bounds__(64 * kGemmWaves, 2) void k_gemm_int4(GemmArgs a) {
     if (!wave_ok) return;
     float* pp = a.part + (size_t)blockIdx.z * a.M * a.N;
 #pragma unroll
-    for (int j = 0; j < kGemmTiles; j++) {
-        const int col = lcol[ws] + 16 * (4 * (wave & 1) + j) + (lane & 15);
+    for (int j = 0; j < GT; j++) {
+        const int col = lcol[ws] + 16 * (GT * (wave & 1) + j) + (lane & 15);
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
@@ -1546,6 +1557,17 @@ __global__ __launch_bounds__(256) void k_gemm_reduce4(const float* __restrict__ 
     }
 }
 
+// plain products over groups of 64 or 32 columns
+template <int RT>
+int launch_gemm_narrow(const GemmArgs& a, dim3 grid, int GT) {
+    const dim3 block(64 * kGemmWaves);
+    if (GT == 2)
+        hipLaunchKernelGGL((k_gemm_int4<RT, 1, kProNone, true, 2>), grid, block, 0, stream(), a);
+    else
+        hipLaunchKernelGGL((k_gemm_int4<RT, 1, kProNone, true, 1>), grid, block, 0, stream(), a);
+    return launch_check("k_gemm_int4");
+}
+
 template <int RT, int NG>
 int launch_gemm(const GemmArgs& a, dim3 grid, bool fold) {
     const dim3 block(64 * kGemmWaves);
@@ -1696,10 +1718,14 @@ extern "C" int cgk_gemm_int4_supported(int M, int K, int N, int gs, int paired) 
 
 // Launch shape of the GEMM over M rows.
 struct GemmPlan {
-    int RT, colblocks, rowblocks, ksteps, ksplit;
+    int RT, GT, colblocks, rowblocks, ksteps, ksplit;
 };
 
-static GemmPlan gemm_plan(int M, int K, int N, int paired) {
+// Column tiles a wave takes: the 2 GT tiles of a slot lie in one scale group
+// (0: a group width that the GEMM does not take).
+static int gemm_tiles(int gs) { return gs % 128 == 0 ? 4 : gs % 64 == 0 ? 2 : gs % 32 == 0 ? 1 : 0; }
+
+static GemmPlan gemm_plan(int M, int K, int N, int gs, int paired) {
     // row tiles per block: up to 3 (48 rows) for short batches; longer ones
     // run as blocks of 2 row tiles (32 rows), which doubles the blocks that
     // share the weights and leaves fewer K splits to reduce (measured on the
@@ -1708,7 +1734,8 @@ static GemmPlan gemm_plan(int M, int K, int N, int paired) {
     const int RT = M > 48 ? 2 : (M + 15) / 16;
     const int BM = 16 * RT;
     const int rowblocks = (M + BM - 1) / BM;
-    const int colblocks = paired ? N / 2 / 128 : (N / 128 + 1) / 2;
+    const int GT = gemm_tiles(gs);
+    const int colblocks = paired ? N / 2 / 128 : (N / (32 * GT) + 1) / 2;
     const int nchunks = K / kChunkK;
     // two blocks per CU, splits of at least two chunks, and partial sums
     // (8 M bytes per column and split, written and read) at most about twice
@@ -1720,7 +1747,7 @@ static GemmPlan gemm_plan(int M, int K, int N, int paired) {
     ksplit = ksplit < 1 ? 1 : (ksplit > 16 ? 16 : ksplit);
     const int ksteps = (nchunks + ksplit - 1) / ksplit;
     ksplit = (nchunks + ksteps - 1) / ksteps;
-    return GemmPlan{RT, colblocks, rowblocks, ksteps, ksplit};
+    return GemmPlan{RT, GT, colblocks, rowblocks, ksteps, ksplit};
 }
 
 // Scratch of the GEMM: the row factors, then the splits' partial sums.
@@ -1734,8 +1761,11 @@ static size_t gemm_row_bytes(int M) { return (((size_t)M * 8) + 255) & ~(size_t)
 //   M 32     2048 x 2048 10.6 / 12.6  4096 x 4096 17.3 / 14.9  11008 x 4096 40 / 21
 //   M 17     4096 x 4096 12.7 / 13.7  4096 x 8192 16.0 / 17.3  11008 x 4096 27 / 20
 //   M 16     4096 x 8192 10.7 / 15.2  11008 x 4096 19.2 / 16.0
+// Groups of 64 and 32 columns cross over at the same rows: M 24 4096 x 4096
+// 19.7 / 16.2 and 20.3 / 16.6, M 32 2048 x 2048 10.9 / 12.0 and 11.4 / 12.1,
+// M 17 11008 x 4096 25.7 / 22.3 and 77 / 25, 4096 x 4096 12.8 / 15.0.
 extern "C" int cgk_gemm_int4_pays(int M, int K, int N, int gs) {
-    if (!cgk_gemm_int4_supported(M, K, N, gs, 0)) return 0;
+    if (M < 1 || K % kChunkK || !gemm_tiles(gs) || N % gs) return 0;
     const size_t kn = (size_t)K * N;
     return M > 48 || (M > 24 && kn >= (size_t)1 << 24) || (M > 16 && kn >= (size_t)5 << 23);
 }
@@ -1749,9 +1779,9 @@ extern "C" int cgk_gemm_int4_max_rows(int K, int N) {
 // 1 when the scratch of a plain GEMM of M rows is at hand: not while the
 // stream is captured (a graph must not keep a scratch address, which a later
 // call's growth frees), nor when the device has no memory for it.
-extern "C" int cgk_gemm_int4_ready(int M, int K, int N) {
+extern "C" int cgk_gemm_int4_ready(int M, int K, int N, int gs) {
     if (cgx_is_capturing()) return 0;
-    const GemmPlan p = gemm_plan(M, K, N, 0);
+    const GemmPlan p = gemm_plan(M, K, N, gs, 0);
     if (cgx_scratch(CGX_SLOT_WS5, gemm_row_bytes(M) +
                                       (p.ksplit > 1 ? (size_t)p.ksplit * M * N * 4 : 0)))
         return 1;
@@ -1765,13 +1795,16 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
                              const float* stats_in, int nstat_in, float* stats_out,
                              const float* nw_next) {
     const int paired = epi == kEpiSwiGlu;
-    if (!cgk_gemm_int4_supported(M, K, N, gs, paired) || ldx < K || (ldx & 3) ||
+    // plain products also over groups of 32 and 64 columns
+    const bool plain = pro == kProNone && epi == kEpiStore && !stats_in && !stats_out;
+    const bool small = plain && M >= 1 && K % kChunkK == 0 && gemm_tiles(gs) && N % gs == 0;
+    if (!(small || cgk_gemm_int4_supported(M, K, N, gs, paired)) || ldx < K || (ldx & 3) ||
         ((uintptr_t)x & 15) || (pro == kProRmsNorm && (!nw || ((uintptr_t)nw & 15))) ||
         ldy < (paired ? N / 2 : N) || (size_t)M * N >= (1u << 31)) {
         cgx_set_error("gemm_int4: unsupported shape M=%d K=%d N=%d gs=%d", M, K, N, gs);
         return -1;
     }
-    const GemmPlan p = gemm_plan(M, K, N, paired);
+    const GemmPlan p = gemm_plan(M, K, N, gs, paired);
     const int RT = p.RT, colblocks = p.colblocks, rowblocks = p.rowblocks;
     const int ksteps = p.ksteps, ksplit = p.ksplit;
     // one split storing plain rows (the lm_head of a tree verify): the GEMM
@@ -1811,14 +1844,17 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
         return -1;
     }
     dim3 grid(colblocks, rowblocks, ksplit);
-    const bool fold = pro == kProNone && epi == kEpiStore && !stats_in && !stats_out;
     int rc;
-    if (paired)
-        rc = RT == 1 ? launch_gemm<1, 2>(a, grid, fold) : RT == 2 ? launch_gemm<2, 2>(a, grid, fold)
-                                                        : launch_gemm<3, 2>(a, grid, fold);
+    if (p.GT != kGemmTiles)
+        rc = RT == 1   ? launch_gemm_narrow<1>(a, grid, p.GT)
+             : RT == 2 ? launch_gemm_narrow<2>(a, grid, p.GT)
+                       : launch_gemm_narrow<3>(a, grid, p.GT);
+    else if (paired)
+        rc = RT == 1 ? launch_gemm<1, 2>(a, grid, plain) : RT == 2 ? launch_gemm<2, 2>(a, grid, plain)
+                                                        : launch_gemm<3, 2>(a, grid, plain);
     else
-        rc = RT == 1 ? launch_gemm<1, 1>(a, grid, fold) : RT == 2 ? launch_gemm<2, 1>(a, grid, fold)
-                                                        : launch_gemm<3, 1>(a, grid, fold);
+        rc = RT == 1 ? launch_gemm<1, 1>(a, grid, plain) : RT == 2 ? launch_gemm<2, 1>(a, grid, plain)
+                                                        : launch_gemm<3, 1>(a, grid, plain);
     if (rc || direct) return rc;
     const int Nout = paired ? N / 2 : N;
     const size_t outs = (size_t)M * Nout;

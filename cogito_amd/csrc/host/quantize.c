@@ -258,7 +258,7 @@ static int matmul_mfma(const float* x, int M, const cg_tensor_quant* w, const cg
         const float* xr = x + (size_t)m0 * K;
         float* yr = y + (size_t)m0 * N;
         int rc;
-        if (cgk_gemm_int4_pays(rows, K, N, gs) && cgk_gemm_int4_ready(rows, K, N))
+        if (cgk_gemm_int4_pays(rows, K, N, gs) && cgk_gemm_int4_ready(rows, K, N, gs))
             rc = cgk_gemm_int4(xr, K, rows, K, N, gs, w->data, w->scales, info->smax, yr, N, 0,
                                NULL, 0.0f, 0, NULL, 0, NULL, NULL);
         else
@@ -287,6 +287,11 @@ int cgx_matmul_int4_dev_kernel(const float* x, int M, cg_tensor_quant* w,
     if (kernel == 3 || kernel == 4) {
         if (info.layout != CGX_LAYOUT_MFMA) {
             cgx_set_error("cgx_matmul_int4: MFMA kernels need a layout-3 weight");
+            return -1;
+        }
+        if (kernel == 4 && !cgk_gemm_int4_supported(M, info.K, info.N, info.group_size, 0)) {
+            cgx_set_error("gemm_int4: unsupported shape M=%d K=%d N=%d gs=%d", M, info.K, info.N,
+                          info.group_size);
             return -1;
         }
         if (kernel == 4)      /* the GEMM of the batched / tree verify (M >= 16) */

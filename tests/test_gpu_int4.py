@@ -117,6 +117,18 @@ def test_matmul_dispatch_by_rows(gpu, oracle, rng, K, N, gs, M):
     _gemv_case(gpu, oracle, rng, K, N, gs, M, 3, 0)
 
 
+@pytest.mark.parametrize("K,N,gs,M", [
+    (256, 64, 64, 49), (256, 96, 32, 49),   # one missing slot, one row block and a row
+    (512, 32, 32, 70), (768, 704, 64, 97), (512, 864, 96, 64), (512, 576, 192, 65),
+    (11008, 4096, 64, 17), (11008, 4096, 32, 33),   # 2 and 3 row tiles, K split
+    (4096, 4096, 32, 24), (4096, 4096, 64, 25),     # either side of the GEMV
+    (512, 336, 48, 70),                     # a group that the GEMM does not take
+])
+def test_matmul_narrow_groups(gpu, oracle, rng, K, N, gs, M):
+    print(f"narrow groups K={K} N={N} gs={gs} M={M}", flush=True)
+    _gemv_case(gpu, oracle, rng, K, N, gs, M, 3, 0)
+
+
 def test_matmul_many_rows_wide_dynamic_range(gpu, oracle, rng):
     # rows of very different magnitudes, a zero row and values spanning many
     # binades through the default dispatch (the GEMM's per-row scaling)
