@@ -685,23 +685,43 @@ __device__ __forceinline__ void chunk_vals(const G& g, int base, int n, float (&
     for (int k = 0; k < kCh; k++) x[k] = (base + k < n) ? g(base + k) : 0.0f;
 }
 
-// raw rows: 16-byte loads when the chunk is whole and aligned (a lane's 32
-// consecutive values in 8 loads rather than 32 strided ones)
-__device__ __forceinline__ void chunk_vals(const RowSrc& g, int base, int n, float (&x)[kCh]) {
-    if (base + kCh <= n && ((uintptr_t)(g.p + base) & 15u) == 0) {
-        const float4* q = reinterpret_cast<const float4*>(g.p + base);
+// kCh consecutive floats in 16-byte loads.  Global loads need 4-byte alignment
+// only, so rows of an odd length (a 50257-value row starts anywhere) take them
+// too: element loads make 64 partial lines an instruction, 32 times, over more
+// lines than the L1 holds.
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_chunk(const float* p, float (&x)[kCh]) {
+    const vf4u* q = reinterpret_cast<const vf4u*>(p);
 #pragma unroll
-        for (int j = 0; j < kCh / 4; j++) {
-            const float4 v = q[j];
-            x[4 * j] = v.x;
-            x[4 * j + 1] = v.y;
-            x[4 * j + 2] = v.z;
-            x[4 * j + 3] = v.w;
-        }
+    for (int j = 0; j < kCh / 4; j++) {
+        const vf4u v = q[j];
+        x[4 * j] = v.x;
+        x[4 * j + 1] = v.y;
+        x[4 * j + 2] = v.z;
+        x[4 * j + 3] = v.w;
+    }
+}
+
+// raw rows: 16-byte loads when the chunk is whole (a lane's 32 consecutive
+// values in 8 loads rather than 32 strided ones)
+__device__ __forceinline__ void chunk_vals(const RowSrc& g, int base, int n, float (&x)[kCh]) {
+    if (base + kCh <= n) {
+        load_chunk(g.p + base, x);
     } else {
 #pragma unroll
         for (int k = 0; k < kCh; k++) x[k] = (base + k < n) ? g.p[base + k] : 0.0f;
     }
+}
+
+// residuals of two raw rows (ResidualGen's operation on the loaded chunks):
+// the corrections of 4 rows of 128256 values 155 -> 70 us, 6 of 50257 72 -> 40
+__device__ __forceinline__ void chunk_vals(const ResidualGen<RowSrc, RowSrc>& g, int base, int n,
+                                           float (&x)[kCh]) {
+    float q[kCh];
+    chunk_vals(g.p, base, n, x);
+    chunk_vals(g.q, base, n, q);
+#pragma unroll
+    for (int k = 0; k < kCh; k++) x[k] = fmaxf(0.0f, __fsub_rn(x[k], q[k]));
 }
 
 // Exact ordered sum of at most two chunks (n <= 64): one wave evaluates the
@@ -835,19 +855,11 @@ __device__ __forceinline__ void load_vals(const S& src, int n, float pad, float 
     for (int k = 0; k < kCh; k++) x[k] = base + k < n ? src(base + k) : pad;
 }
 
-// raw rows: 16-byte loads where the thread's 32 elements are whole and aligned
+// raw rows: 16-byte loads where the thread's 32 elements are whole
 __device__ __forceinline__ void load_vals(const RowSrc& src, int n, float pad, float (&x)[kCh]) {
     const int base = threadIdx.x * kCh;
-    if (base + kCh <= n && ((uintptr_t)src.p & 15u) == 0) {
-        const float4* q = reinterpret_cast<const float4*>(src.p + base);
-#pragma unroll
-        for (int j = 0; j < kCh / 4; j++) {
-            const float4 v = q[j];
-            x[4 * j] = v.x;
-            x[4 * j + 1] = v.y;
-            x[4 * j + 2] = v.z;
-            x[4 * j + 3] = v.w;
-        }
+    if (base + kCh <= n) {
+        load_chunk(src.p + base, x);
     } else {
 #pragma unroll
         for (int k = 0; k < kCh; k++) x[k] = base + k < n ? src.p[base + k] : pad;

@@ -277,6 +277,9 @@ def test_filtered_verify_batch_device(gpu, oracle, rng):
     (2, 33000, 3, 1.0, 50, 1.0),            # long rows' candidate pass, unscaled
     (2, 33000, 3, 0.7, 50, 0.9),            # and scaled
     (5, 500, 7, 1.0, 0, 0.8),
+    (1, 70001, 1, 1.5, 0, 0.999),           # a nucleus that ends in the third round
+    (1, 40001, 1, 1.0, 0, 0.9999999),       # one that no bound ends before the row
+    (2, 50257, 1, 0.7, 0, 0.95),            # rows that start at any 4-byte address
 ])
 def test_filtered_verify_rows_of_both_arrays(gpu, oracle, rng, B, V, gamma, T, k, p):
     """Target and draft rows share the filter's launches: every chain of a batch
