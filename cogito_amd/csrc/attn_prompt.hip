@@ -43,7 +43,8 @@ namespace {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
@@ -203,12 +204,14 @@ __global__ __launch_bounds__(kThreads) void k_prompt_pack(PackArgs a) {
 }
 
 // Maximum / sum over the four lane groups (lanes 16 and 32 apart).  The
-// maximum as the bare instruction: fmaxf first quiets values that come from a
-// lane exchange.
+// maximum as a median with an infinity that the compiler cannot see: fmaxf
+// first quiets values that come from a lane exchange.  No instruction here is written in inline asm: between an
+// MFMA and a write of its C operand the hardware needs wait states, which the
+// compiler inserts only around instructions that it knows.
 __device__ __forceinline__ float max2(float a, float b) {
-    float r;
-    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    float inf = __builtin_inff();
+    asm("" : "+s"(inf));
+    return __builtin_amdgcn_fmed3f(a, b, inf);
 }
 __device__ __forceinline__ float groups_max(float v) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -223,22 +226,21 @@ __device__ __forceinline__ float groups_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// split8 with the conversions back to fp32 as instructions of their own: the
-// compiler's v_fma_mix for the remainder runs at half rate.
+// split8 with the conversions back to fp32 as instructions of their own (the
+// empty asm hides the value's origin): the compiler's v_fma_mix for the
+// remainder runs at half rate.
 __device__ __forceinline__ void split8_fast(const float (&v)[8], f16x8& hi, f16x8& lo) {
-    uint32_t h[4], l[4];
+    f16x2 h[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        float a, b;
-        asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(h[i]) : "v"(v[2 * i]), "v"(v[2 * i + 1]));
-        asm("v_cvt_f32_f16 %0, %1" : "=v"(a) : "v"(h[i]));
-        asm("v_cvt_f32_f16_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1"
-            : "=v"(b) : "v"(h[i]));
-        const float ra = v[2 * i] - a, rb = v[2 * i + 1] - b;
-        asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(l[i]) : "v"(ra), "v"(rb));
+        h[i] = __builtin_convertvector((f32x2){v[2 * i], v[2 * i + 1]}, f16x2);
+        float a = (float)h[i][0], b = (float)h[i][1];
+        asm volatile("" : "+v"(a), "+v"(b));
+        l[i] = __builtin_convertvector((f32x2){v[2 * i] - a, v[2 * i + 1] - b}, f16x2);
     }
-    hi = __builtin_bit_cast(f16x8, (u32x4){h[0], h[1], h[2], h[3]});
-    lo = __builtin_bit_cast(f16x8, (u32x4){l[0], l[1], l[2], l[3]});
+    hi = __builtin_bit_cast(f16x8, h);
+    lo = __builtin_bit_cast(f16x8, l);
+    asm volatile("" : "+v"(lo));
 }
 
 // Barrier that orders LDS accesses only: the next tile's loads stay in flight.
