@@ -185,7 +185,7 @@ struct AttnArgs {
     float* part_ml;              // [splits][B][Nq][H][2]
     float* lse;                  // optional [B][H][Nq] (splits == 1)
     // run only where *only_if == gen (nullptr: always): the second pass over
-    // inputs that the packed path found not to be finite
+    // inputs that the packed path does not take
     const unsigned* only_if;
     unsigned gen;
 };

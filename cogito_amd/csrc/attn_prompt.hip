@@ -76,7 +76,7 @@ struct PackArgs {
     const float* K;              // [B][Nk][Hk][D]
     const float* V;
     int B, Nk, Hk, D, tiles;     // tiles: records per (sequence, KV head)
-    unsigned* flag;              // set to `gen` when a value is not finite
+    unsigned* flag;              // set to `gen` by an input that k_attn has to take
     unsigned gen;
     uint8_t* rec;
 };
@@ -95,7 +95,7 @@ struct PromptArgs {
     float* part_o;               // [splits][B*Nq*H][D]
     float* part_ml;              // [splits][B*Nq*H][2]
     float* lse;                  // [B][H][Nq] or nullptr
-    unsigned* flag;
+    unsigned* flag;              // as in PackArgs
     unsigned gen;
 };
 
@@ -107,6 +107,16 @@ __device__ __forceinline__ int key_of_pos(int p) {
     const int g = p >> 3, j = p & 7;
     return j < 4 ? 4 * g + j : 16 + 4 * g + j - 4;
 }
+
+// Ends of the range of row maxima that the packed path takes; other inputs run
+// k_attn (see PromptArgs::flag).  Q times scale and K below 2^50: a score in a
+// row's held units, without Q's power of two, stays below 2^74.  V from 2^-100
+// (or zero): a key's weight times its V multiplier is no subnormal.  A Q row is
+// scaled up by at most 2^60: the lowest value, -FLT_MAX in held units, stands
+// for a score below -2^67, so that a hidden key weighs nothing beside a visible
+// one, and a score of queries too small for the scaling is off by at most 2^-28.
+constexpr float kMaxQK = 0x1p50f, kMinV = 0x1p-100f;
+constexpr int kMaxQExp = 60;
 
 // Exponent e such that |v| * 2^e < 2^15 for |v| <= m, m finite (m = 0: 0).
 __device__ __forceinline__ int scale_exp(float m) {
@@ -154,12 +164,12 @@ __global__ __launch_bounds__(kThreads) void k_prompt_pack(PackArgs a) {
             // x * 0 is NaN for an infinity or a NaN
             bad += kv[i][j] * 0.0f + vv[i][j] * 0.0f;
         }
-    if (bad != bad) *a.flag = a.gen;
 #pragma unroll
     for (int o = 1; o < 8; o <<= 1) {
         km = fmaxf(km, __shfl_xor(km, o));
         vm = fmaxf(vm, __shfl_xor(vm, o));
     }
+    if (bad != bad || km >= kMaxQK || (vm > 0.0f && vm < kMinV)) *a.flag = a.gen;
     const int ek = scale_exp(km), ev = scale_exp(vm);
 #pragma unroll
     for (int i = 0; i < UPT; i++)
@@ -348,7 +358,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
                 bad += qv[c][j] * 0.0f;
             }
         m = groups_max(m);
-        const int e = scale_exp(m);
+        if (m >= kMaxQK) bad = __builtin_nanf("");
+        const int e = min(scale_exp(m), kMaxQExp);
         qmul[rt] = ldexpf(1.0f, -e);
 #pragma unroll
         for (int c = 0; c < CB; c++) {
@@ -359,8 +370,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     }
     if (bad != bad) *a.flag = a.gen;
 
-    // scores are held without the row's Q multiplier (a power of two): x times
-    // qmul is the score, and the softmax's exponent is (x - m) qmul log2(e)
+    // scores are held without the row's Q multiplier (a power of two), under a
+    // custom mask, which any value may enter, as they are: x times unit is the
+    // score, and the softmax's exponent is (x - m) unit log2(e)
+    auto unit = [&](int rt) { return a.mask_kind == kMaskCustom ? 1.0f : qmul[rt]; };
     float m_run[RT], l_run[RT];
     int er[RT];                    // O is held times 2^(141 - er)
     f32x4 o[RT][TD];
@@ -452,13 +465,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
                 if (a.mask_kind == kMaskAligned) vis = kk <= nk - a.Nq + q;
                 else if (a.mask_kind == kMaskTL) vis = kk <= q;
                 else if (a.mask_kind == kMaskWindow) vis = abs(kk - q) <= a.window;
-                else if (a.mask_kind == kMaskCustom && kk < nk) {
-                    // the score with the mask added, back in the held units
-                    // (an infinite one stays so, a finite one stays finite)
-                    const float sc = v * qmul[rt] + a.mask[(size_t)q * nk + kk];
-                    v = sc / qmul[rt];
-                    if (fabsf(sc) <= FLT_MAX) v = fminf(fmaxf(v, -FLT_MAX), FLT_MAX);
-                }
+                else if (a.mask_kind == kMaskCustom && kk < nk)
+                    v = v * qmul[rt] + a.mask[(size_t)q * nk + kk];
                 x[rt][j] = kk >= nk ? -__builtin_inff() : (vis ? v : -FLT_MAX);
             }
     };
@@ -488,7 +496,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
             float f[RT];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
-                const float c = qmul[rt] * 1.44269504088896340736f;
+                const float c = unit(rt) * 1.44269504088896340736f;
                 float mx = m_run[rt];
 #pragma unroll
                 for (int j = 0; j < 8; j++) mx = fmaxf(mx, x[rt][j]);
@@ -564,7 +572,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     for (int rt = 0; rt < RT; rt++) {
         const float L = groups_sum(l_run[rt]);
         // the row's maximum score (a masked one stays the lowest value)
-        const float M = m_run[rt] > -FLT_MAX ? m_run[rt] * qmul[rt] : m_run[rt];
+        const float M = m_run[rt] > -FLT_MAX ? m_run[rt] * unit(rt) : m_run[rt];
         const size_t orow = ((size_t)b * a.Nq + rq[rt]) * a.H + rh[rt];
         const float down = ldexpf(1.0f, er[rt] - 141);
         float* dst = a.splits == 1 ? a.O + orow * a.D : a.part_o + ((size_t)split * nrow + orow) * a.D;
@@ -643,7 +651,7 @@ extern "C" int cgx_flash_packed_min(int mega) {
 }
 
 // Flash forward (every mask of cgk_attention but the tree's).  *flag receives
-// *gen when an input is not finite: the caller then runs the fp32 kernel over
+// *gen when an input is not finite or outside the ranges above: the caller then runs the fp32 kernel over
 // the same output, whose products are the reference's.  Returns 0, -1 on an
 // error, or 1 when the call has to take the fp32 kernel (no scratch memory, a
 // grid too large, stream capture).

@@ -240,8 +240,9 @@ int cgk_attn_dec_batch(const float* Q, const uint8_t* kc, const uint8_t* vc, con
 /* fp32 flash attention of many query rows (attn_prompt.hip), K and V packed
  * once per call into MFMA operands.  pays: whether the call's size repays the
  * packing.  f32 returns 0, -1 on an error, or 1 when the call has to take the
- * fp32 kernel; afterwards *flag holds *gen when an input was not finite, and
- * the fp32 kernel then has to run over the same output. */
+ * fp32 kernel; afterwards *flag holds *gen when an input was not finite or
+ * outside the exponents that the path takes, and the fp32 kernel then has to
+ * run over the same output. */
 int cgk_attn_prompt_pays(int B, int Nq, int Nk, int H, int Hk, int D);
 int cgk_attn_prompt_f32(const float* Q, const float* K, const float* V, int B, int Nq, int Nk,
                         int H, int Hk, int D, float scale, int mask_kind, int window,

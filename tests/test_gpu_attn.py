@@ -485,6 +485,82 @@ def test_flash_packed_magnitudes(gpu, oracle, rng, packed_always):
     assert rel_err_rows(O.reshape(-1, 64), eO.reshape(-1, 64)) <= TOL
 
 
+def attention64(Q, K, V, scale, mt, W=0, mask=None):
+    """Attention in 64 bits over scores rounded to fp32 once, to which a custom
+    mask is added in fp32 (a mask of -1e38 swallows its score, as in fp32)."""
+    B, Nq, H, D = Q.shape
+    Nk, Hk = K.shape[1], K.shape[2]
+    kv = np.arange(H) * Hk // H
+    k, v = K[:, :, kv].astype(np.float64), V[:, :, kv].astype(np.float64)
+    x = np.einsum("bqhd,bkhd->bhqk", Q.astype(np.float64) * scale, k).astype(np.float32)
+    q, j = np.arange(Nq)[:, None], np.arange(Nk)[None]
+    if mt == 1:
+        x = np.where(j <= q, x, -FLT_MAX)
+    elif mt == 2:
+        x = np.where(np.abs(j - q) <= W, x, -FLT_MAX)
+    elif mt == 3:
+        x = x + mask
+    x = x.astype(np.float64)
+    m = x.max(-1, keepdims=True)
+    e = np.exp(x - np.where(np.isinf(m), 0.0, m))
+    L = e.sum(-1, keepdims=True)
+    O = np.einsum("bhqk,bkhd->bqhd", np.divide(e, L, out=np.zeros_like(e), where=L > 0), v)
+    with np.errstate(divide="ignore"):
+        return O, (m + np.log(L))[..., 0]
+
+
+# of a row's largest value: a product of two hi + lo operands is off by at most
+# 2^-21 of itself, and 128 of them with scores of a few units by less than 2e-6
+PACKED_TOL = 5e-6
+
+
+def check_packed(gpu, Q, K, V, mt, W=0, mask=None):
+    D = Q.shape[3]
+    O, lse, p = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, mt, W, mask)
+    eO, el = attention64(Q, K, V, p.scale, mt, W, mask)
+    assert np.all(np.isfinite(O))
+    assert rel_err_rows(O.reshape(-1, D), eO.reshape(-1, D)) <= PACKED_TOL
+    fin = np.isfinite(el)
+    np.testing.assert_allclose(lse[fin], el[fin].astype(np.float32), rtol=PACKED_TOL, atol=1e-5)
+    np.testing.assert_array_equal(lse[~fin], el[~fin].astype(np.float32))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mt,W", [(1, 0), (2, 9)])
+def test_flash_packed_hidden_keys_at_any_query_size(gpu, rng, packed_always, mt, W, D):
+    # a hidden key has no weight however small the row's queries are (their
+    # scores then all are about 0: the weight of a key that leaked would be 1)
+    Q, K, V = attn_inputs(rng, 1, 70, 70, 4, 2, D)
+    e = np.array([0, -30, -60, -64, -90, -104, -110, -112, -116, -120, -124, -130, -140])
+    Q = (Q * np.exp2(e[(np.arange(70)[:, None] + 3 * np.arange(4)) % e.size])[None, :, :, None])
+    Q[:, 33] = 0.0
+    check_packed(gpu, Q.astype(np.float32), K, V, mt, W)
+
+
+def test_flash_packed_custom_masks_down_to_the_lowest_value(gpu, rng, packed_always):
+    # the largest of several very low mask values takes a row's whole weight,
+    # and lse reports it; equal ones share it; rows of -inf alone give zeros
+    Q, K, V = attn_inputs(rng, 1, 40, 50, 2, 2, 64)
+    low = np.float32([-1e33, -2e34, -1e35, -1e38, -3e38, -FLT_MAX])
+    mask = rng.choice(low, (40, 50)).astype(np.float32)
+    mask[3] = -np.inf
+    mask[4] = np.where(np.arange(50) % 2, -FLT_MAX, np.float32(-1e38))
+    mask[5], mask[6], mask[7] = -FLT_MAX, np.float32(-1e38), np.float32(1e38)
+    mask[8] = np.where(np.arange(50) < 30, -np.inf, np.float32(-5e37))
+    mask[9, ::3] = 0.0
+    check_packed(gpu, Q, K, V, 3, 0, mask)
+
+
+@pytest.mark.parametrize("eq,ek,ev", [(0, 108, 0), (-100, 102, 0), (-20, 124, 0), (102, -100, 0),
+                                      (49, 52, 0), (0, 0, 122), (0, 0, -126), (-60, 45, 0),
+                                      (-146, -20, 0)])
+def test_flash_packed_far_exponents(gpu, rng, packed_always, eq, ek, ev):
+    # finite inputs whose scores are finite, at the ends of the exponent range
+    Q, K, V = attn_inputs(rng, 1, 40, 90, 4, 2, 64)
+    Q, K, V = ((x * np.exp2(float(e))).astype(np.float32) for x, e in ((Q, eq), (K, ek), (V, ev)))
+    check_packed(gpu, Q, K, V, 1)
+
+
 @pytest.mark.parametrize("where", ["q", "k", "v"])
 def test_flash_packed_non_finite_inputs(gpu, rng, where):
     # infinities and NaN give what the fp32 kernel gives, bit for bit, and
