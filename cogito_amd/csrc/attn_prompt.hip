@@ -679,19 +679,16 @@ extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* 
     if (Hk > 65535 || chunks * B > 65535 || R + 128 > 0x7fffffff) return 1;
     const long long first = blocks * splits <= 512 ? 256 / (splits * Hk * B) : chunks;
     const size_t nrow = (size_t)B * Nq * H;
-    pk.rec = (uint8_t*)cgx_scratch(CGX_SLOT_WS4, (size_t)(4 * (DP / 32) * P + 1) * kBlock * tiles *
-                                                     Hk * B);
+    pk.rec = (uint8_t*)cgx_scratch_try(CGX_SLOT_WS4, (size_t)(4 * (DP / 32) * P + 1) * kBlock *
+                                                         tiles * Hk * B);
     unsigned* f = cgx_counters(1);
     bool room = pk.rec && f;
     if (room && splits > 1) {
-        a.part_o = (float*)cgx_scratch(CGX_SLOT_WS2, (size_t)splits * nrow * D * 4);
-        a.part_ml = (float*)cgx_scratch(CGX_SLOT_WS3, (size_t)splits * nrow * 2 * 4);
+        a.part_o = (float*)cgx_scratch_try(CGX_SLOT_WS2, (size_t)splits * nrow * D * 4);
+        a.part_ml = (float*)cgx_scratch_try(CGX_SLOT_WS3, (size_t)splits * nrow * 2 * 4);
         room = a.part_o && a.part_ml;
     }
-    if (!room) {
-        cgx_clear_error();         // the fp32 kernel needs less
-        return 1;
-    }
+    if (!room) return 1;           // the fp32 kernel needs less
     if (++g_gen == 0) g_gen = 1;
     pk.K = K; pk.V = V;
     pk.B = a.B = B;

@@ -26,6 +26,10 @@ enum { CGX_SLOT_IN0 = 0, CGX_SLOT_IN1, CGX_SLOT_IN2, CGX_SLOT_IN3,
        CGX_SLOT_WS2, CGX_SLOT_WS3, CGX_SLOT_WS4, CGX_SLOT_WS5, CGX_SLOT_WS6,
        CGX_NUM_SLOTS };
 void* cgx_scratch(int slot, size_t bytes);
+/* The same for a caller that can do without: NULL where the device has no
+ * memory for it, or the buffer would grow under stream capture, and the
+ * library's error is left alone. */
+void* cgx_scratch_try(int slot, size_t bytes);
 /* 1 while the library stream is being captured into a graph. */
 int cgx_is_capturing(void);
 /* Zero-initialised counters that kernels reset themselves after use. */

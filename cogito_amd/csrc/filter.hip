@@ -1024,11 +1024,9 @@ static size_t top_p_bytes(int rows, int V, size_t* wsb) {
 extern "C" int cgk_filter_rows_fit(int rows, int V, int top_k) {
     if (rows > 65535) return 0;
     size_t wsb;
-    void* p = top_k > 0 && top_k < V
-                  ? cgx_scratch(CGX_SLOT_WS6, topk_bytes(rows))
-                  : cgx_scratch(CGX_SLOT_WS0, top_p_bytes(rows, V, &wsb));
-    if (!p) cgx_clear_error();
-    return p != nullptr;
+    return (top_k > 0 && top_k < V
+                ? cgx_scratch_try(CGX_SLOT_WS6, topk_bytes(rows))
+                : cgx_scratch_try(CGX_SLOT_WS0, top_p_bytes(rows, V, &wsb))) != nullptr;
 }
 
 // The same over rows of two arrays at once: na rows of x (whose rows draw the

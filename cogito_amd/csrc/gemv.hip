@@ -1782,11 +1782,9 @@ extern "C" int cgk_gemm_int4_max_rows(int K, int N) {
 extern "C" int cgk_gemm_int4_ready(int M, int K, int N, int gs) {
     if (cgx_is_capturing()) return 0;
     const GemmPlan p = gemm_plan(M, K, N, gs, 0);
-    if (cgx_scratch(CGX_SLOT_WS5, gemm_row_bytes(M) +
-                                      (p.ksplit > 1 ? (size_t)p.ksplit * M * N * 4 : 0)))
-        return 1;
-    cgx_clear_error();             // the GEMV needs none
-    return 0;
+    return cgx_scratch_try(CGX_SLOT_WS5, gemm_row_bytes(M) +
+                                             (p.ksplit > 1 ? (size_t)p.ksplit * M * N * 4 : 0)) !=
+           nullptr;
 }
 
 extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs,

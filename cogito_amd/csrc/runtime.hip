@@ -25,6 +25,7 @@ struct Runtime {
     hipEvent_t events[8] = {};
     void* scratch[CGX_NUM_SLOTS] = {};
     size_t scratch_bytes[CGX_NUM_SLOTS] = {};
+    size_t scratch_limit = 0;               // test hook (0: none)
     unsigned int* counters = nullptr;
     size_t counter_count = 0;
 };
@@ -129,6 +130,7 @@ extern "C" void* cgx_malloc(size_t bytes) {
     void* p = nullptr;
     hipError_t e = hipMalloc(&p, bytes ? bytes : 1);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // else the next launch check reports it
         cgx_set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         return nullptr;
     }
@@ -307,35 +309,67 @@ extern "C" int cgx_graph_free(void* graph) {
     return 0;
 }
 
-extern "C" void* cgx_scratch(int slot, size_t bytes) {
-    if (cgx_ensure_init()) return nullptr;
-    if (slot < 0 || slot >= CGX_NUM_SLOTS) {
-        cgx_set_error("cgx_scratch: bad slot %d", slot);
-        return nullptr;
-    }
+// A slot's buffer of at least `bytes`; nullptr where the device has no memory
+// for it, with *e the allocator's error, which is cleared (HIP keeps the last
+// error until it is read, and the next launch check would report it).
+static void* scratch_get(int slot, size_t bytes, size_t* want_out, hipError_t* e) {
+    *e = hipSuccess;
     if (bytes > g_rt.scratch_bytes[slot]) {
-        if (capturing("cgx_scratch (growth)")) return nullptr;
         size_t want = bytes < 4096 ? 4096 : bytes + bytes / 4;
+        if (g_rt.scratch_limit && want > g_rt.scratch_limit) want = (size_t)1 << 50;
+        *want_out = want;
         if (g_rt.scratch[slot]) {
-            if (hipStreamSynchronize(g_rt.stream) != hipSuccess ||
-                hipFree(g_rt.scratch[slot]) != hipSuccess) {
-                cgx_set_error("cgx_scratch: releasing slot %d failed", slot);
+            if ((*e = hipStreamSynchronize(g_rt.stream)) != hipSuccess ||
+                (*e = hipFree(g_rt.scratch[slot])) != hipSuccess)
                 return nullptr;
-            }
         }
         g_rt.scratch[slot] = nullptr;
         g_rt.scratch_bytes[slot] = 0;
         void* p = nullptr;
-        hipError_t e = hipMalloc(&p, want);
-        if (e != hipSuccess) {
-            cgx_set_error("cgx_scratch: hipMalloc(%zu) failed: %s", want,
-                          hipGetErrorString(e));
+        if ((*e = hipMalloc(&p, want)) != hipSuccess) {
+            (void)hipGetLastError();
             return nullptr;
         }
         g_rt.scratch[slot] = p;
         g_rt.scratch_bytes[slot] = want;
     }
     return g_rt.scratch[slot];
+}
+
+extern "C" void* cgx_scratch(int slot, size_t bytes) {
+    if (cgx_ensure_init()) return nullptr;
+    if (slot < 0 || slot >= CGX_NUM_SLOTS) {
+        cgx_set_error("cgx_scratch: bad slot %d", slot);
+        return nullptr;
+    }
+    if (bytes > g_rt.scratch_bytes[slot] && capturing("cgx_scratch (growth)")) return nullptr;
+    size_t want = 0;
+    hipError_t e;
+    void* p = scratch_get(slot, bytes, &want, &e);
+    if (!p && e != hipSuccess)
+        cgx_set_error("cgx_scratch: slot %d, %zu bytes: %s", slot, want, hipGetErrorString(e));
+    return p;
+}
+
+extern "C" void* cgx_scratch_try(int slot, size_t bytes) {
+    if (cgx_ensure_init() || slot < 0 || slot >= CGX_NUM_SLOTS) return nullptr;
+    if (bytes > g_rt.scratch_bytes[slot] && cgx_is_capturing()) return nullptr;
+    size_t want = 0;
+    hipError_t e;
+    return scratch_get(slot, bytes, &want, &e);
+}
+
+extern "C" size_t cgx_scratch_limit(size_t bytes) {
+    const size_t old = g_rt.scratch_limit;
+    if (cgx_ensure_init()) return old;
+    g_rt.scratch_limit = bytes;
+    for (int i = 0; bytes && i < CGX_NUM_SLOTS; i++) {
+        if (g_rt.scratch_bytes[i] <= bytes) continue;
+        if (hipStreamSynchronize(g_rt.stream) == hipSuccess) (void)hipFree(g_rt.scratch[i]);
+        g_rt.scratch[i] = nullptr;
+        g_rt.scratch_bytes[i] = 0;
+    }
+    return old;
 }
 
 extern "C" unsigned int* cgx_counters(size_t count) {
@@ -356,6 +390,7 @@ extern "C" unsigned int* cgx_counters(size_t count) {
         if (hipMalloc(&p, want * sizeof(unsigned int)) != hipSuccess ||
             hipMemset(p, 0, want * sizeof(unsigned int)) != hipSuccess ||
             hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
             cgx_set_error("cgx_counters: allocation of %zu counters failed", want);
             return nullptr;
         }

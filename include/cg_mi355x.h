@@ -311,6 +311,10 @@ int cgx_gemm_swiglu_here(int on);
  * KV heads * rows * keys * head_dim (default 150; 0 always); returns the
  * previous value (-1 only reads it). */
 int cgx_flash_packed_min(int mega);
+/* Test hook, no reference counterpart: scratch buffers above this many bytes
+ * are asked of the device as one that it cannot have, and larger ones held
+ * are released (0, the default: no limit); returns the previous limit. */
+size_t cgx_scratch_limit(size_t bytes);
 int cgx_attention_int4_kv_batch_dev(const float* Q, int B, int Nq, int H,
                                     cg_kv_cache_int4* cache, int slot0, const int* nk,
                                     int mask_kind, const unsigned long long* anc, int tw,
