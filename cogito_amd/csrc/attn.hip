@@ -184,10 +184,6 @@ struct AttnArgs {
     float* part_o;               // [splits][B][Nq][H][D]
     float* part_ml;              // [splits][B][Nq][H][2]
     float* lse;                  // optional [B][H][Nq] (splits == 1)
-    // run only where *only_if == gen (nullptr: always): the second pass over
-    // inputs that the packed path does not take
-    const unsigned* only_if;
-    unsigned gen;
 };
 
 __device__ __forceinline__ int head_begin(int hk, int H, int Hk) { return (hk * H + Hk - 1) / Hk; }
@@ -204,7 +200,6 @@ __global__ __launch_bounds__(256) void k_attn(AttnArgs a) {
     __shared__ float sP[4][32][33];     // per-wave S, then P, tile
     __shared__ float sM[4][32], sL[4][32], sAlpha[4][32];
 
-    if (a.only_if && *a.only_if != a.gen) return;      // uniform over the grid
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int split = blockIdx.x;
     const int hk = blockIdx.y % a.Hk, b = blockIdx.y / a.Hk;
@@ -581,15 +576,6 @@ extern "C" int cgk_attention(const float* Q, int int4, const uint8_t* kc, const 
     if (int4 && !lse && aligned && cgk_attn_dec_supported(D, gs, B, mask_kind))
         return cgk_attn_dec(Q, kc, vc, ks, vs, Nq, Nk, H, Hk, D, scale, mask_kind, anc, O);
     AttnArgs a;
-    a.only_if = nullptr;
-    a.gen = 0;
-    if (!int4 && mask_kind != kMaskTree && (mask_kind != kMaskCausal || Nk >= Nq) &&
-        cgk_attn_prompt_pays(B, Nq, Nk, H, Hk, D)) {
-        const int rc = cgk_attn_prompt_f32(Q, K, V, B, Nq, Nk, H, Hk, D, scale, mask_kind, window,
-                                           mask, O, lse, &a.only_if, &a.gen);
-        if (rc < 0) return -1;
-        if (rc > 0) a.only_if = nullptr;
-    }
     a.Q = Q; a.int4 = int4; a.kc = kc; a.vc = vc; a.ks = ks; a.vs = vs; a.gs = gs;
     a.K = K; a.V = V; a.B = B; a.Nq = Nq; a.Nk = Nk; a.H = H; a.Hk = Hk; a.D = D;
     a.scale = scale; a.mask_kind = mask_kind; a.window = window; a.mask = mask;
@@ -603,7 +589,7 @@ extern "C" int cgk_attention(const float* Q, int int4, const uint8_t* kc, const 
     int chunks = (max_g * Nq + 31) / 32;
     // enough blocks to fill 256 CUs twice, at least 128 keys (4 tiles) per split
     long long base_blocks = (long long)Hk * B * chunks;
-    int splits = a.only_if ? 1 : (int)((512 + base_blocks - 1) / base_blocks);
+    int splits = (int)((512 + base_blocks - 1) / base_blocks);
     int max_splits = (Nk + 127) / 128;
     if (splits > max_splits) splits = max_splits;
     if (splits < 1) splits = 1;

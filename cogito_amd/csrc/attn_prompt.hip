@@ -27,7 +27,8 @@
 // Rows are ordered by position, heads fastest, so that a block's causal range
 // ends early; tiles that no row of the block sees are skipped.  Measured at
 // that size: 724 us for k_attn (scalar K loads a row apart, every tile of the
-// causal mask), 82 us for the call here (pack 10, attention 65, second pass 4).
+// causal mask), 78 us for the call here (pack 10, attention 65).  A call whose
+// inputs the operands cannot hold costs this time before k_attn's.
 // The VALU's share bounds it: about 175 instructions a wave and tile beside 48
 // MFMAs.
 #include <hip/hip_runtime.h>
@@ -62,7 +63,7 @@ int launch_check(const char* what) {
     return 0;
 }
 
-enum { kMaskNone = 0, kMaskAligned = 1, kMaskWindow = 2, kMaskCustom = 3, kMaskTL = 5 };
+enum { kMaskNone = 0, kMaskWindow = 2, kMaskCustom = 3, kMaskCausal = 5 };   // CGK_MASK_*
 
 constexpr int P = 2;                      // parts of a value: hi, lo
 // Blocks of a record: K fragments [key half][32-dim chunk][part], the keys' K
@@ -76,8 +77,7 @@ struct PackArgs {
     const float* K;              // [B][Nk][Hk][D]
     const float* V;
     int B, Nk, Hk, D, tiles;     // tiles: records per (sequence, KV head)
-    unsigned* flag;              // set to `gen` by an input that k_attn has to take
-    unsigned gen;
+    unsigned* flag;              // set by an input that k_attn has to take
     uint8_t* rec;
 };
 
@@ -96,10 +96,15 @@ struct PromptArgs {
     float* part_ml;              // [splits][B*Nq*H][2]
     float* lse;                  // [B][H][Nq] or nullptr
     unsigned* flag;              // as in PackArgs
-    unsigned gen;
 };
 
 __device__ __forceinline__ int head_begin(int hk, int H, int Hk) { return (hk * H + Hk - 1) / Hk; }
+
+// The flag is a word of host memory, written by the first inputs of a call that
+// k_attn has to take, read once the stream is idle.
+__device__ __forceinline__ void refuse(unsigned* flag) {
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Position p (0..31) of a V fragment row holds this key of the tile: the keys
 // whose scores a lane of group p / 8 holds after S^T = K Q^T.
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(kThreads) void k_prompt_pack(PackArgs a) {
         km = fmaxf(km, __shfl_xor(km, o));
         vm = fmaxf(vm, __shfl_xor(vm, o));
     }
-    if (bad != bad || km >= kMaxQK || (vm > 0.0f && vm < kMinV)) *a.flag = a.gen;
+    if (bad != bad || km >= kMaxQK || (vm > 0.0f && vm < kMinV)) refuse(a.flag);
     const int ek = scale_exp(km), ev = scale_exp(vm);
 #pragma unroll
     for (int i = 0; i < UPT; i++)
@@ -292,8 +297,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     const int rlast = min(row0 + 16 * RT * kWaves, R) - 1;
     const int qa = row0 / G, qb = rlast / G;
     int klo = 0, khi = nk;
-    if (a.mask_kind == kMaskAligned) khi = min(nk, nk - a.Nq + qb + 1);
-    if (a.mask_kind == kMaskTL) khi = min(nk, qb + 1);
+    if (a.mask_kind == kMaskCausal) khi = min(nk, qb + 1);
     // (a row that sees no key averages all of them, as in the reference)
     if (a.mask_kind == kMaskWindow && a.window >= 0 && qb - a.window < nk) {
         klo = max(0, qa - a.window);
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
             split8(qv[c], qh[rt][c], ql[rt][c]);
         }
     }
-    if (bad != bad) *a.flag = a.gen;
+    if (bad != bad) refuse(a.flag);
 
     // scores are held without the row's Q multiplier (a power of two), under a
     // custom mask, which any value may enter, as they are: x times unit is the
@@ -391,8 +395,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     const int qmin = wr0 / G, qmax = wr1 / G;
     // the last tile that some row of this wave sees
     int tw1 = t1;
-    if (a.mask_kind == kMaskAligned) tw1 = min(t1, (nk - a.Nq + qmax) / kTile + 1);
-    if (a.mask_kind == kMaskTL) tw1 = min(t1, qmax / kTile + 1);
+    if (a.mask_kind == kMaskCausal) tw1 = min(t1, qmax / kTile + 1);
 
     f32x4 s[RT][2], sx[RT][2];
     auto scores = [&](int buf) {
@@ -439,8 +442,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
         const int kt = t * kTile;
         bool full = kt + kTile <= nk;
         switch (a.mask_kind) {
-            case kMaskAligned: full = full && kt + kTile - 1 <= nk - a.Nq + qmin; break;
-            case kMaskTL: full = full && kt + kTile - 1 <= qmin; break;
+            case kMaskCausal: full = full && kt + kTile - 1 <= qmin; break;
             case kMaskWindow:
                 full = full && (long long)kt >= (long long)qmax - a.window &&
                        (long long)kt + kTile - 1 <= (long long)qmin + a.window;
@@ -462,8 +464,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
                 const int q = rq[rt];
                 bool vis = true;
                 float v = x[rt][j];
-                if (a.mask_kind == kMaskAligned) vis = kk <= nk - a.Nq + q;
-                else if (a.mask_kind == kMaskTL) vis = kk <= q;
+                if (a.mask_kind == kMaskCausal) vis = kk <= q;
                 else if (a.mask_kind == kMaskWindow) vis = abs(kk - q) <= a.window;
                 else if (a.mask_kind == kMaskCustom && kk < nk)
                     v = v * qmul[rt] + a.mask[(size_t)q * nk + kk];
@@ -621,7 +622,7 @@ int launch_all(const PackArgs& pk, PromptArgs& a, int RT) {
     return launch_check("k_prompt_attn");
 }
 
-unsigned g_gen = 0;       // a new mark for each call's non-finite flag
+unsigned* g_flag = nullptr;    // host memory that the kernels write (PackArgs::flag)
 int g_min_mega = 150;     // the packed path's least work (cgk_attn_prompt_pays), in 1e6
 
 }  // namespace
@@ -650,15 +651,11 @@ extern "C" int cgx_flash_packed_min(int mega) {
     return old;
 }
 
-// Flash forward (every mask of cgk_attention but the tree's).  *flag receives
-// *gen when an input is not finite or outside the ranges above: the caller then runs the fp32 kernel over
-// the same output, whose products are the reference's.  Returns 0, -1 on an
-// error, or 1 when the call has to take the fp32 kernel (no scratch memory, a
-// grid too large, stream capture).
+// Flash forward.  Returns 0, -1 on an error, or 1 when the call has to take
+// k_attn (no scratch memory, a grid too large, stream capture).
 extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* V, int B, int Nq,
                                    int Nk, int H, int Hk, int D, float scale, int mask_kind,
-                                   int window, const float* mask, float* O, float* lse,
-                                   const unsigned** flag, unsigned* gen) {
+                                   int window, const float* mask, float* O, float* lse) {
     if (cgx_is_capturing()) return 1;
     const int DP = (D + 31) / 32 * 32, tiles = (Nk + kTile - 1) / kTile;
     const long long R = (long long)((H + Hk - 1) / Hk) * Nq;
@@ -681,23 +678,26 @@ extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* 
     const size_t nrow = (size_t)B * Nq * H;
     pk.rec = (uint8_t*)cgx_scratch_try(CGX_SLOT_WS4, (size_t)(4 * (DP / 32) * P + 1) * kBlock *
                                                          tiles * Hk * B);
-    unsigned* f = cgx_counters(1);
-    bool room = pk.rec && f;
+    if (!g_flag && hipHostMalloc((void**)&g_flag, 64, hipHostMallocCoherent) != hipSuccess) {
+        (void)hipGetLastError();
+        g_flag = nullptr;
+    }
+    bool room = pk.rec && g_flag;
     if (room && splits > 1) {
         a.part_o = (float*)cgx_scratch_try(CGX_SLOT_WS2, (size_t)splits * nrow * D * 4);
         a.part_ml = (float*)cgx_scratch_try(CGX_SLOT_WS3, (size_t)splits * nrow * 2 * 4);
         room = a.part_o && a.part_ml;
     }
     if (!room) return 1;           // the fp32 kernel needs less
-    if (++g_gen == 0) g_gen = 1;
+    // no earlier call's kernels run any more: each is waited for (flash_run)
+    *(volatile unsigned*)g_flag = 0;
     pk.K = K; pk.V = V;
     pk.B = a.B = B;
     pk.Nk = a.Nk = Nk;
     pk.Hk = a.Hk = Hk;
     pk.D = a.D = D;
     pk.tiles = a.tiles = tiles;
-    pk.flag = a.flag = f;
-    pk.gen = a.gen = g_gen;
+    pk.flag = a.flag = g_flag;
     a.Q = Q; a.Nq = Nq; a.H = H;
     a.rec = pk.rec;
     a.scale = scale;
@@ -708,10 +708,10 @@ extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* 
     a.vec = D == DP && !((uintptr_t)O & 15);
     a.O = O;
     a.lse = lse;
-    *flag = f;
-    *gen = g_gen;
     const int rc = DP == 64 ? launch_all<64>(pk, a, RT)
                  : DP == 96 ? launch_all<96>(pk, a, RT) : launch_all<128>(pk, a, RT);
     if (rc || splits == 1) return rc;
     return cgk_attn_combine(a.part_o, a.part_ml, (int)splits, (int)nrow, D, Nq, H, O, lse);
 }
+
+extern "C" int cgk_attn_prompt_refused(void) { return *(volatile unsigned*)g_flag != 0; }

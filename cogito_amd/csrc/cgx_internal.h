@@ -32,8 +32,6 @@ void* cgx_scratch(int slot, size_t bytes);
 void* cgx_scratch_try(int slot, size_t bytes);
 /* 1 while the library stream is being captured into a graph. */
 int cgx_is_capturing(void);
-/* Zero-initialised counters that kernels reset themselves after use. */
-unsigned int* cgx_counters(size_t count);
 /* Device view of a host-or-device argument: returns p itself when it is a
  * device pointer, else copies `bytes` into scratch `slot`. */
 const void* cgx_dev_in(const void* p, size_t bytes, int slot);
@@ -243,15 +241,16 @@ int cgk_attn_dec_batch(const float* Q, const uint8_t* kc, const uint8_t* vc, con
 
 /* fp32 flash attention of many query rows (attn_prompt.hip), K and V packed
  * once per call into MFMA operands.  pays: whether the call's size repays the
- * packing.  f32 returns 0, -1 on an error, or 1 when the call has to take the
- * fp32 kernel; afterwards *flag holds *gen when an input was not finite or
- * outside the exponents that the path takes, and the fp32 kernel then has to
- * run over the same output. */
+ * packing.  f32 (mask kinds none, window, custom and causal) returns 0, -1 on
+ * an error, or 1 when the call has to take cgk_attention.  refused, once the
+ * library stream is idle: whether an input of the last such call was not
+ * finite or outside the exponents that the path takes; its output is then
+ * cgk_attention's to write. */
 int cgk_attn_prompt_pays(int B, int Nq, int Nk, int H, int Hk, int D);
 int cgk_attn_prompt_f32(const float* Q, const float* K, const float* V, int B, int Nq, int Nk,
                         int H, int Hk, int D, float scale, int mask_kind, int window,
-                        const float* mask, float* O, float* lse, const unsigned** flag,
-                        unsigned* gen);
+                        const float* mask, float* O, float* lse);
+int cgk_attn_prompt_refused(void);
 /* Merge of key splits: part_o [splits][nrow][D] and part_ml [splits][nrow][2]
  * (maximum, sum) into O, and lse where given. */
 int cgk_attn_combine(const float* part_o, const float* part_ml, int splits, int nrow, int D,

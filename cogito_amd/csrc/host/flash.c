@@ -8,6 +8,7 @@
  * call returns.  All-device calls return after the GPU finished.
  */
 #include <math.h>
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -18,6 +19,11 @@
 /* Device view of an input array: the pointer itself, or a scratch copy. */
 static const float* dev_view(const float* p, size_t n, int slot) {
     return (const float*)cgx_dev_in(p, n * sizeof(float), slot);
+}
+
+/* Whether [a, a + na) and [b, b + nb) floats share memory. */
+static int overlap(const float* a, size_t na, const float* b, size_t nb) {
+    return a && b && (uintptr_t)a < (uintptr_t)(b + nb) && (uintptr_t)b < (uintptr_t)(a + na);
 }
 
 /* Runs attention for params with KV head count Hk and kernel mask kind. */
@@ -48,9 +54,23 @@ static void flash_run(const char* who, cg_flash_attn_params* p, int Hk, int kind
     float* dlse = NULL;
     if (p->softmax_lse) dlse = ld ? p->softmax_lse : (float*)cgx_scratch(CGX_SLOT_OUT1, nl * 4);
     if (!dout || (p->softmax_lse && !dlse)) return;
-    if (cgk_attention(dq, 0, NULL, NULL, NULL, NULL, 0, dk, dv, B, Nq, Nk, H, Hk, D, p->scale,
-                      kind, p->window_size, dm, NULL, dout, dlse))
-        return;
+    /* The packed path, where its size pays; then cgk_attention for a call that
+     * it refuses, or whose inputs it found that it cannot hold (known once it
+     * has run, so an output over an input goes to cgk_attention at once). */
+    const size_t nm = (size_t)Nq * Nk;
+    const int in_place = overlap(dout, nq, dq, nq) || overlap(dout, nq, dk, nk) ||
+                         overlap(dout, nq, dv, nk) || overlap(dout, nq, dm, nm) ||
+                         overlap(dlse, nl, dq, nq) || overlap(dlse, nl, dk, nk) ||
+                         overlap(dlse, nl, dv, nk) || overlap(dlse, nl, dm, nm);
+    int rc = 1;
+    if (!in_place && cgk_attn_prompt_pays(B, Nq, Nk, H, Hk, D))
+        rc = cgk_attn_prompt_f32(dq, dk, dv, B, Nq, Nk, H, Hk, D, p->scale, kind, p->window_size,
+                                 dm, dout, dlse);
+    if (rc == 0) rc = cgx_synchronize() ? -1 : cgk_attn_prompt_refused();
+    if (rc > 0)
+        rc = cgk_attention(dq, 0, NULL, NULL, NULL, NULL, 0, dk, dv, B, Nq, Nk, H, Hk, D, p->scale,
+                           kind, p->window_size, dm, NULL, dout, dlse);
+    if (rc) return;
     if (!od && cgx_memcpy_d2h(p->O, dout, nq * sizeof(float))) return;
     if (p->softmax_lse && !ld && cgx_memcpy_d2h(p->softmax_lse, dlse, nl * 4)) return;
     if (od && ld) cgx_synchronize();

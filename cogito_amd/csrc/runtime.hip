@@ -26,8 +26,6 @@ struct Runtime {
     void* scratch[CGX_NUM_SLOTS] = {};
     size_t scratch_bytes[CGX_NUM_SLOTS] = {};
     size_t scratch_limit = 0;               // test hook (0: none)
-    unsigned int* counters = nullptr;
-    size_t counter_count = 0;
 };
 
 Runtime g_rt;
@@ -370,34 +368,6 @@ extern "C" size_t cgx_scratch_limit(size_t bytes) {
         g_rt.scratch_bytes[i] = 0;
     }
     return old;
-}
-
-extern "C" unsigned int* cgx_counters(size_t count) {
-    if (cgx_ensure_init()) return nullptr;
-    if (count > g_rt.counter_count) {
-        if (capturing("cgx_counters (growth)")) return nullptr;
-        size_t want = count < 4096 ? 4096 : count;
-        if (g_rt.counters) {
-            if (hipStreamSynchronize(g_rt.stream) != hipSuccess ||
-                hipFree(g_rt.counters) != hipSuccess) {
-                cgx_set_error("cgx_counters: release failed");
-                return nullptr;
-            }
-        }
-        g_rt.counters = nullptr;
-        g_rt.counter_count = 0;
-        void* p = nullptr;
-        if (hipMalloc(&p, want * sizeof(unsigned int)) != hipSuccess ||
-            hipMemset(p, 0, want * sizeof(unsigned int)) != hipSuccess ||
-            hipDeviceSynchronize() != hipSuccess) {
-            (void)hipGetLastError();
-            cgx_set_error("cgx_counters: allocation of %zu counters failed", want);
-            return nullptr;
-        }
-        g_rt.counters = (unsigned int*)p;
-        g_rt.counter_count = want;
-    }
-    return g_rt.counters;
 }
 
 extern "C" const void* cgx_dev_in(const void* p, size_t bytes, int slot) {

@@ -586,6 +586,33 @@ def test_flash_packed_non_finite_inputs(gpu, rng, where):
     np.testing.assert_array_equal(_bits(al), _bits(bl))
 
 
+@pytest.mark.parametrize("kind", ["finite", "inf", "far"])
+@pytest.mark.parametrize("splits", [1, 4])
+def test_flash_output_over_its_queries(gpu, rng, packed_always, kind, splits):
+    # an output that shares memory with the queries: the result of separate
+    # buffers, also where the inputs are left to the fp32 kernel
+    Nq, Nk, H, D = 32, 40 if splits == 1 else 500, 2, 64
+    Q, K, V = attn_inputs(rng, 1, Nq, Nk, H, H, D)
+    if kind == "inf":
+        Q[0, 3, 0, 0] = np.inf
+    elif kind == "far":
+        K[0, 5] *= np.float32(1e30)
+        Q *= np.float32(1e-30)
+    out = []
+    for shared, mega in ((False, 1 << 30), (True, 0)):
+        gpu.cgx_flash_packed_min(mega)
+        dq, dk, dv = (DeviceArray.from_numpy(gpu, x) for x in (Q, K, V))
+        o = dq if shared else DeviceArray(gpu, Q.nbytes)
+        p = CgFlashAttnParams(Q=dq.ptr, K=dk.ptr, V=dv.ptr, O=o.ptr, batch_size=1, seqlen_q=Nq,
+                              seqlen_k=Nk, n_heads=H, n_heads_k=H, d_head=D, scale=0.125,
+                              mask_type=0)
+        gpu.cgx_clear_error()
+        gpu.cg_flash_attention_forward(C.byref(p))
+        assert last_error(gpu) in ("", None), last_error(gpu)
+        out.append(o.numpy(np.float32, Q.shape))
+    np.testing.assert_array_equal(out[0], out[1])
+
+
 def test_flash_forward_device_pointers(gpu, oracle, rng):
     B, Nq, Nk, H, Hk, D = 1, 50, 50, 4, 2, 64
     Q, K, V = attn_inputs(rng, B, Nq, Nk, H, Hk, D)
