@@ -10,27 +10,31 @@
 // fragments: per (sequence, KV head, 32-key tile) a record of 1 KiB blocks, a
 // block holding the 16 bytes of each lane in lane order, so that the attention
 // copies a record linearly and reads LDS without bank conflicts.  A value
-// becomes hi + lo fp16, each rounded to nearest, after a power-of-two scaling
-// per key row: an error of at most 2^-24 of the value, one fp32 rounding.
-// k_prompt_attn then runs 64 RT query rows a block (4 waves of 16 RT rows) over
-// the tiles of one KV head: scores S^T = K Q^T and O^T = V^T P^T on
-// v_mfma_f32_16x16x32_f16, Q and P as hi + lo fp16 (P times its key's V
+// becomes hi + lo / 2^12 fp16, each rounded to nearest, after a power-of-two
+// scaling per key row: off by at most 2^-23 of itself or 2^-52 of the row's
+// maximum.  k_prompt_attn then runs 64 query rows a block (4 waves of 16 rows)
+// over the tiles of one KV head: scores S^T = K Q^T and O^T = V^T P^T on
+// v_mfma_f32_16x16x32_f16, Q and P as such pairs too (P times its key's V
 // multiplier, scaled by a power of two that follows the largest contribution of
-// each query row), products hi hi + hi lo + lo hi, sums in fp32.  Three such
-// products cost 3/16 of one on the fp32 matrix instructions, and 32 products
-// are summed per rounding instead of 2: the error against 64 bits is below that
-// of k_attn's fp32 products (1021 causal rows of 32 heads over 8 of 128: 2.4e-7
-// against 3.3e-7; over all shapes above head_dim 32 measured, 2.7e-7 to 3.4e-7
-// against 3.1e-7 to 4.7e-7).  In the S^T orientation a lane holds one query row
-// and 8 keys of a tile, which is the B operand of P^T: P never moves.
+// each query row), the products hi hi in one fp32 sum, hi lo + lo hi in
+// another, added at the end (lo lo, at most 2^-22 of the product, is left out).
+// Three such products cost 3/16 of one on the fp32 matrix instructions, and 32
+// products are summed per rounding instead of 2: the error against 64 bits is
+// below that of k_attn's fp32 products (1021 causal rows of 32 heads over 8 of
+// 128: 1.9e-7 against 3.2e-7; 1000 rows of 12 heads of 64 over 1900 keys 2.8e-7
+// against 4.1e-7; 700 windowed rows of 16/2 heads of 96 2.1e-7 against 3.6e-7).
+// lo times 2^12 and its own sums cost 2 us of 80 at the first of these sizes;
+// without them a value below 2^-17 of its row's maximum loses bits (dims of O
+// 2^-30 of the others': an error of 3e-3).  In the S^T orientation a lane holds
+// one query row and 8 keys of a tile, which is the B operand of P^T: P never
+// moves.
 //
 // Rows are ordered by position, heads fastest, so that a block's causal range
 // ends early; tiles that no row of the block sees are skipped.  Measured at
 // that size: 724 us for k_attn (scalar K loads a row apart, every tile of the
-// causal mask), 78 us for the call here (pack 10, attention 65).  A call whose
-// inputs the operands cannot hold costs this time before k_attn's.
-// The VALU's share bounds it: about 175 instructions a wave and tile beside 48
-// MFMAs.
+// causal mask), 80 us for the call here.  A call whose inputs the operands
+// cannot hold costs this time before k_attn's.  The VALU's share bounds it:
+// about 175 instructions a wave and tile beside 48 MFMAs.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -129,12 +133,13 @@ __device__ __forceinline__ int scale_exp(float m) {
     return m > 0.0f ? 141 - (ex > 1 ? ex : 1) : 0;             // 2^(ex-127) <= m < 2^(ex-126)
 }
 
-// hi + lo fp16 of 8 values, each rounded to nearest.
+// hi + lo / kLo fp16 of 8 values below 2^15, each rounded to nearest.
+constexpr float kLo = 4096.0f;             // |v - hi| <= 2^3: lo stays in range
 __device__ __forceinline__ void split8(const float (&v)[8], f16x8& hi, f16x8& lo) {
 #pragma unroll
     for (int i = 0; i < 8; i++) hi[i] = (_Float16)v[i];
 #pragma unroll
-    for (int i = 0; i < 8; i++) lo[i] = (_Float16)(v[i] - (float)hi[i]);
+    for (int i = 0; i < 8; i++) lo[i] = (_Float16)((v[i] - (float)hi[i]) * kLo);
 }
 
 // One block per (32-key tile, KV head, sequence).  A thread takes 8-dim units
@@ -220,9 +225,10 @@ __global__ __launch_bounds__(kThreads) void k_prompt_pack(PackArgs a) {
 
 // Maximum / sum over the four lane groups (lanes 16 and 32 apart).  The
 // maximum as a median with an infinity that the compiler cannot see: fmaxf
-// first quiets values that come from a lane exchange.  No instruction here is written in inline asm: between an
-// MFMA and a write of its C operand the hardware needs wait states, which the
-// compiler inserts only around instructions that it knows.
+// first quiets values that come from a lane exchange.  No instruction here is
+// written in inline asm: between an MFMA and a write of its C operand the
+// hardware needs wait states, which the compiler inserts only around
+// instructions that it knows.
 __device__ __forceinline__ float max2(float a, float b) {
     float inf = __builtin_inff();
     asm("" : "+s"(inf));
@@ -251,7 +257,8 @@ __device__ __forceinline__ void split8_fast(const float (&v)[8], f16x8& hi, f16x
         h[i] = __builtin_convertvector((f32x2){v[2 * i], v[2 * i + 1]}, f16x2);
         float a = (float)h[i][0], b = (float)h[i][1];
         asm volatile("" : "+v"(a), "+v"(b));
-        l[i] = __builtin_convertvector((f32x2){v[2 * i] - a, v[2 * i + 1] - b}, f16x2);
+        l[i] = __builtin_convertvector(
+            (f32x2){(v[2 * i] - a) * kLo, (v[2 * i + 1] - b) * kLo}, f16x2);
     }
     hi = __builtin_bit_cast(f16x8, h);
     lo = __builtin_bit_cast(f16x8, l);
@@ -265,13 +272,19 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+constexpr float kGrow = 8.0f;              // in binades
+
 // Each iteration runs the products of the next tile's scores beside the
 // softmax of this tile's, which do not depend on each other, so that the
 // matrix cores and the VALU work at the same time within a wave (the call at
-// the size above 91 us with one tile at a time, 84 with its operand reads
-// grouped, 82 so).  LDS holds the K part of tile t + 1 and the V part
-// of tile t, both double buffered, behind one barrier a tile.
-template <int DP, int RT>
+// the size above, before lo had sums of its own, 91 us with one tile at a time,
+// 84 with its operand reads grouped, 82 so).  LDS holds the K part of tile
+// t + 1 and the V part of tile t, both double buffered, behind one barrier a
+// tile.  O is rescaled only where a row's maximum grows by more than kGrow or
+// its contributions leave the room kept for them (83 -> 80 us).  128 rows a
+// block do not fit the registers (head_dim 64, 4 x 1021 causal rows of 32
+// heads: 175 us with spills, 164 with 64 rows).
+template <int DP>
 __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     constexpr int CB = DP / 32, TD = DP / 16;
     constexpr int NB = kRecBlocks<DP>;              // 1 KiB blocks of a record
@@ -290,11 +303,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
     const int nk = a.Nk;
     const int h0 = head_begin(hk, a.H, a.Hk), G = head_begin(hk + 1, a.H, a.Hk) - h0;
     const int R = G * a.Nq;
-    const int row0 = chunk * 16 * RT * kWaves;
+    const int row0 = chunk * 16 * kWaves;
     if (row0 >= R) return;                             // uniform over the block
 
     // ---- the block's rows and the tiles they see
-    const int rlast = min(row0 + 16 * RT * kWaves, R) - 1;
+    const int rlast = min(row0 + 16 * kWaves, R) - 1;
     const int qa = row0 / G, qb = rlast / G;
     int klo = 0, khi = nk;
     if (a.mask_kind == kMaskCausal) khi = min(nk, qb + 1);
@@ -337,67 +350,53 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
         fetch_v(t0);
     }
 
-    // ---- Q operands: row 16 (RT wave + rt) + n of the block, scaled, hi + lo
-    f16x8 qh[RT][CB], ql[RT][CB];
-    float qmul[RT];
-    int rq[RT], rh[RT];
-    bool rok[RT];
-    float bad = 0.0f;
+    // ---- Q operands: row 16 wave + n of the block, scaled, hi + lo
+    f16x8 qh[CB], ql[CB];
+    const int r = row0 + 16 * wave + n;
+    const bool rok = r < R;
+    const int rq = (rok ? r : rlast) / G, rh = h0 + (rok ? r : rlast) % G;
+    const float* qp = a.Q + (((size_t)b * a.Nq + rq) * a.H + rh) * a.D;
+    float qv[CB][8];
+    float m = 0.0f, bad = 0.0f;
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-        const int r = row0 + 16 * (RT * wave + rt) + n;
-        rok[rt] = r < R;
-        rq[rt] = (rok[rt] ? r : rlast) / G;
-        rh[rt] = h0 + (rok[rt] ? r : rlast) % G;
-        const float* qp = a.Q + (((size_t)b * a.Nq + rq[rt]) * a.H + rh[rt]) * a.D;
-        float qv[CB][8];
-        float m = 0.0f;
+    for (int c = 0; c < CB; c++)
 #pragma unroll
-        for (int c = 0; c < CB; c++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int d = 32 * c + 8 * g + j;
-                qv[c][j] = d < a.D ? qp[d] * a.scale : 0.0f;
-                m = fmaxf(m, fabsf(qv[c][j]));
-                bad += qv[c][j] * 0.0f;
-            }
-        m = groups_max(m);
-        if (m >= kMaxQK) bad = __builtin_nanf("");
-        const int e = min(scale_exp(m), kMaxQExp);
-        qmul[rt] = ldexpf(1.0f, -e);
-#pragma unroll
-        for (int c = 0; c < CB; c++) {
-#pragma unroll
-            for (int j = 0; j < 8; j++) qv[c][j] = ldexpf(qv[c][j], e);
-            split8(qv[c], qh[rt][c], ql[rt][c]);
+        for (int j = 0; j < 8; j++) {
+            const int d = 32 * c + 8 * g + j;
+            qv[c][j] = d < a.D ? qp[d] * a.scale : 0.0f;
+            m = fmaxf(m, fabsf(qv[c][j]));
+            bad += qv[c][j] * 0.0f;
         }
+    m = groups_max(m);
+    if (m >= kMaxQK) bad = __builtin_nanf("");
+    const int e = min(scale_exp(m), kMaxQExp);
+    const float qmul = ldexpf(1.0f, -e);
+#pragma unroll
+    for (int c = 0; c < CB; c++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) qv[c][j] = ldexpf(qv[c][j], e);
+        split8(qv[c], qh[c], ql[c]);
     }
     if (bad != bad) refuse(a.flag);
 
     // scores are held without the row's Q multiplier (a power of two), under a
     // custom mask, which any value may enter, as they are: x times unit is the
     // score, and the softmax's exponent is (x - m) unit log2(e)
-    auto unit = [&](int rt) { return a.mask_kind == kMaskCustom ? 1.0f : qmul[rt]; };
-    float m_run[RT], l_run[RT];
-    int er[RT];                    // O is held times 2^(141 - er)
-    f32x4 o[RT][TD];
-    float x[RT][8];                // this tile's scores
+    const float unit = a.mask_kind == kMaskCustom ? 1.0f : qmul;
+    float m_run = -__builtin_inff(), l_run = 0.0f;
+    int er = 16;                   // O is held times 2^(141 - er)
+    f32x4 o[TD], ox[TD];           // products hi hi; hi lo + lo hi, times kLo
+    float x[8];                    // this tile's scores
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-        m_run[rt] = -__builtin_inff();
-        l_run[rt] = 0.0f;
-        er[rt] = 16;
-#pragma unroll
-        for (int t = 0; t < TD; t++) o[rt][t] = (f32x4)(0.0f);
-    }
+    for (int t = 0; t < TD; t++) o[t] = ox[t] = (f32x4)(0.0f);
     // the wave's first and last query positions (mask-free tiles)
-    const int wr0 = min(row0 + 16 * RT * wave, rlast), wr1 = min(wr0 + 16 * RT - 1, rlast);
+    const int wr0 = min(row0 + 16 * wave, rlast), wr1 = min(wr0 + 15, rlast);
     const int qmin = wr0 / G, qmax = wr1 / G;
     // the last tile that some row of this wave sees
     int tw1 = t1;
     if (a.mask_kind == kMaskCausal) tw1 = min(t1, qmax / kTile + 1);
 
-    f32x4 s[RT][2], sx[RT][2];
+    f32x4 s[2], sx[2];
     auto scores = [&](int buf) {
         f16x8 kf[2][CB][P];
 #pragma unroll
@@ -408,24 +407,18 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
                 for (int p = 0; p < P; p++)
                     kf[i][c][p] = ((const f16x8*)(s_k[buf] + ((i * CB + c) * P + p) * kBlock))[lane];
 #pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) s[rt][i] = sx[rt][i] = (f32x4)(0.0f);
+        for (int i = 0; i < 2; i++) s[i] = sx[i] = (f32x4)(0.0f);
 #pragma unroll
         for (int c = 0; c < CB; c++) {
 #pragma unroll
             for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int rt = 0; rt < RT; rt++)
-                    s[rt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[i][c][0], qh[rt][c], s[rt][i], 0, 0, 0);
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[i][c][0], qh[c], s[i], 0, 0, 0);
 #pragma unroll
             for (int p = 0; p < P; p++)
 #pragma unroll
                 for (int i = 0; i < 2; i++)
-#pragma unroll
-                    for (int rt = 0; rt < RT; rt++)
-                        sx[rt][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            kf[i][c][p], p ? qh[rt][c] : ql[rt][c], sx[rt][i], 0, 0, 0);
+                    sx[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                        kf[i][c][p], p ? qh[c] : ql[c], sx[i], 0, 0, 0);
         }
     };
     // the K (0) or V (1) multipliers of the tile in K buffer `buf`
@@ -451,25 +444,21 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
             default: break;
         }
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                x[rt][j] = (s[rt][j >> 2][j & 3] + sx[rt][j >> 2][j & 3]) * kmu[j];
+        for (int j = 0; j < 8; j++)
+            x[j] = fmaf(sx[j >> 2][j & 3], 1.0f / kLo, s[j >> 2][j & 3]) * kmu[j];
         if (full) return;
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int kk = kt + (j < 4 ? 4 * g + j : 12 + 4 * g + j);
-                const int q = rq[rt];
-                bool vis = true;
-                float v = x[rt][j];
-                if (a.mask_kind == kMaskCausal) vis = kk <= q;
-                else if (a.mask_kind == kMaskWindow) vis = abs(kk - q) <= a.window;
-                else if (a.mask_kind == kMaskCustom && kk < nk)
-                    v = v * qmul[rt] + a.mask[(size_t)q * nk + kk];
-                x[rt][j] = kk >= nk ? -__builtin_inff() : (vis ? v : -FLT_MAX);
-            }
+        for (int j = 0; j < 8; j++) {
+            const int kk = kt + (j < 4 ? 4 * g + j : 12 + 4 * g + j);
+            const int q = rq;
+            bool vis = true;
+            float v = x[j];
+            if (a.mask_kind == kMaskCausal) vis = kk <= q;
+            else if (a.mask_kind == kMaskWindow) vis = abs(kk - q) <= a.window;
+            else if (a.mask_kind == kMaskCustom && kk < nk)
+                v = v * qmul + a.mask[(size_t)q * nk + kk];
+            x[j] = kk >= nk ? -__builtin_inff() : (vis ? v : -FLT_MAX);
+        }
     };
 
     float vmu[8];                  // this tile's V multipliers
@@ -493,47 +482,48 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
         if (t < tw1) {             // (beyond it every row of this wave is masked)
             // ---- the next tile's products beside this tile's softmax
             scores(buf ^ 1);
-            f16x8 ph[RT], pl[RT];
-            float f[RT];
+            f16x8 ph, pl;
+            const float c = unit * 1.44269504088896340736f;
+            float mx = m_run;
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                const float c = unit(rt) * 1.44269504088896340736f;
-                float mx = m_run[rt];
+            for (int j = 0; j < 8; j++) mx = fmaxf(mx, x[j]);
+            // a maximum that has grown by no more than kGrow keeps its
+            // place (weights up to 2^kGrow), and O its scale
+            const float m_top = groups_max(mx);
+            const float m_new = (m_top - m_run) * c > kGrow ? m_top : m_run;
+            const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
+            const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * c);
+            float sum = 0.0f, pm = 0.0f;
+            float y[8];
 #pragma unroll
-                for (int j = 0; j < 8; j++) mx = fmaxf(mx, x[rt][j]);
-                const float m_new = groups_max(mx);
-                const float m_use = m_new == -__builtin_inff() ? 0.0f : m_new;
-                const float alpha = __builtin_amdgcn_exp2f((m_run[rt] - m_use) * c);
-                float sum = 0.0f, pm = 0.0f;
-                float y[8];
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float p = __builtin_amdgcn_exp2f((x[rt][j] - m_use) * c);
-                    sum += p;
-                    y[j] = p * vmu[j];
-                    pm = fmaxf(pm, fabsf(y[j]));
-                }
-                l_run[rt] = l_run[rt] * alpha + sum;
-                m_run[rt] = m_new;
-                pm = groups_max(pm);
-                // scale of the row's contributions: the tile's largest, or
-                // what earlier ones have decayed to
-                const int ex = min((int)(__float_as_uint(pm) >> 23), 254);
-                const int ea = (int)(__float_as_uint(alpha) >> 23) - 127 + (alpha < 1.0f ? 1 : 0);
-                const int en = max(max(ex, er[rt] + ea), 16);
-                f[rt] = ldexpf(alpha, er[rt] - en);
-                er[rt] = en;
-                const float up = ldexpf(1.0f, 141 - en);
-#pragma unroll
-                for (int j = 0; j < 8; j++) y[j] *= up;
-                split8_fast(y, ph[rt], pl[rt]);
+            for (int j = 0; j < 8; j++) {
+                const float p = __builtin_amdgcn_exp2f((x[j] - m_use) * c);
+                sum += p;
+                y[j] = p * vmu[j];
+                pm = fmaxf(pm, fabsf(y[j]));
             }
+            l_run = l_run * alpha + sum;
+            m_run = m_new;
+            pm = groups_max(pm);
+            // scale of the row's contributions: what earlier ones have
+            // decayed to, or the tile's largest with room for 3 bits more
+            const int ex = min((int)(__float_as_uint(pm) >> 23), 254);
+            const int ea = (int)(__float_as_uint(alpha) >> 23) - 127 + (alpha < 1.0f ? 1 : 0);
+            const int eo = max(er + ea, 16);
+            const int en = ex > eo ? ex + 3 : eo;
+            const float f = ldexpf(alpha, er - en);
+            er = en;
+            const float up = ldexpf(1.0f, 141 - en);
 #pragma unroll
-            for (int rt = 0; rt < RT; rt++)
-                if (__ballot(f[rt] != 1.0f)) {
+            for (int j = 0; j < 8; j++) y[j] *= up;
+            split8_fast(y, ph, pl);
+            if (__ballot(f != 1.0f)) {
 #pragma unroll
-                    for (int tt = 0; tt < TD; tt++) o[rt][tt] *= f[rt];
+                for (int tt = 0; tt < TD; tt++) {
+                    o[tt] *= f;
+                    ox[tt] *= f;
                 }
+            }
             // ---- O += P V; products of one accumulator stand four apart
             const uint8_t* vb = s_v[buf];
 #pragma unroll
@@ -548,12 +538,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
                 for (int p = 0; p < P + 1; p++)
 #pragma unroll
                     for (int i = 0; i < 4; i++)
-#pragma unroll
-                        for (int rt = 0; rt < RT; rt++)
-                            if (t4 + i < TD)
-                                o[rt][t4 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                    vf[i][p == 2 ? P - 1 : 0], p == 1 ? pl[rt] : ph[rt],
-                                    o[rt][t4 + i], 0, 0, 0);
+                        if (t4 + i < TD) {
+                            f32x4& acc = p ? ox[t4 + i] : o[t4 + i];
+                            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                vf[i][p == 2 ? P - 1 : 0], p == 1 ? pl : ph, acc, 0, 0, 0);
+                        }
             }
         }
         // (nobody reads these buffers before the next barrier)
@@ -569,56 +558,47 @@ __global__ __launch_bounds__(kThreads, 2) void k_prompt_attn(PromptArgs a) {
 
     // ---- O rows: lane (n, g) holds dims 16 tt + 4 g .. + 3 of its rows
     const size_t nrow = (size_t)a.B * a.Nq * a.H;
+    const float L = groups_sum(l_run);
+    // the row's maximum score (a masked one stays the lowest value)
+    const float M = m_run > -FLT_MAX ? m_run * unit : m_run;
+    const size_t orow = ((size_t)b * a.Nq + rq) * a.H + rh;
+    const float down = ldexpf(1.0f, er - 141);
+    float* dst = a.splits == 1 ? a.O + orow * a.D : a.part_o + ((size_t)split * nrow + orow) * a.D;
 #pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-        const float L = groups_sum(l_run[rt]);
-        // the row's maximum score (a masked one stays the lowest value)
-        const float M = m_run[rt] > -FLT_MAX ? m_run[rt] * unit(rt) : m_run[rt];
-        const size_t orow = ((size_t)b * a.Nq + rq[rt]) * a.H + rh[rt];
-        const float down = ldexpf(1.0f, er[rt] - 141);
-        float* dst = a.splits == 1 ? a.O + orow * a.D : a.part_o + ((size_t)split * nrow + orow) * a.D;
+    for (int tt = 0; tt < TD; tt++) {
+        float v[4];
 #pragma unroll
-        for (int tt = 0; tt < TD; tt++) {
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                v[i] = o[rt][tt][i] * down;
-                if (a.splits == 1) v[i] = L > 0.0f ? v[i] / L : 0.0f;
-            }
-            const int d = 16 * tt + 4 * g;
-            if (!rok[rt]) continue;
-            if (a.vec) {
-                *(float4*)(dst + d) = make_float4(v[0], v[1], v[2], v[3]);
-            } else {
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (d + i < a.D) dst[d + i] = v[i];
-            }
+        for (int i = 0; i < 4; i++) {
+            v[i] = fmaf(ox[tt][i], 1.0f / kLo, o[tt][i]) * down;
+            if (a.splits == 1) v[i] = L > 0.0f ? v[i] / L : 0.0f;
         }
-        if (a.splits == 1) {
-            if (rok[rt] && g == 0 && a.lse) {
-                a.lse[((size_t)b * a.H + rh[rt]) * a.Nq + rq[rt]] =
-                    L > 0.0f ? M + logf(L) : -__builtin_inff();
-            }
-        } else if (rok[rt] && g == 0) {
-            *(float2*)&a.part_ml[((size_t)split * nrow + orow) * 2] = make_float2(M, L);
+        const int d = 16 * tt + 4 * g;
+        if (!rok) continue;
+        if (a.vec) {
+            *(float4*)(dst + d) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (d + i < a.D) dst[d + i] = v[i];
         }
+    }
+    if (a.splits == 1) {
+        if (rok && g == 0 && a.lse) {
+            a.lse[((size_t)b * a.H + rh) * a.Nq + rq] =
+                L > 0.0f ? M + logf(L) : -__builtin_inff();
+        }
+    } else if (rok && g == 0) {
+        *(float2*)&a.part_ml[((size_t)split * nrow + orow) * 2] = make_float2(M, L);
     }
 }
 
 template <int DP>
-int launch_all(const PackArgs& pk, PromptArgs& a, int RT) {
+int launch_all(const PackArgs& pk, const PromptArgs& a) {
     hipLaunchKernelGGL(k_prompt_pack<DP>, dim3(pk.tiles, pk.Hk, pk.B), dim3(kThreads), 0, stream(),
                        pk);
     if (launch_check("k_prompt_pack")) return -1;
-    const dim3 grid(a.splits, a.Hk, a.chunks * a.B);
-    if constexpr (DP <= 64) {
-        if (RT == 2) {
-            hipLaunchKernelGGL((k_prompt_attn<DP, 2>), grid, dim3(kThreads), 0, stream(), a);
-            return launch_check("k_prompt_attn");
-        }
-    }
-    hipLaunchKernelGGL((k_prompt_attn<DP, 1>), grid, dim3(kThreads), 0, stream(), a);
+    hipLaunchKernelGGL(k_prompt_attn<DP>, dim3(a.splits, a.Hk, a.chunks * a.B), dim3(kThreads), 0,
+                       stream(), a);
     return launch_check("k_prompt_attn");
 }
 
@@ -628,18 +608,19 @@ int g_min_mega = 150;     // the packed path's least work (cgk_attn_prompt_pays)
 }  // namespace
 
 // Whether the packed path takes an attention over fp32 K/V.  It costs a pass
-// over K and V and a third launch; k_attn's time grows with the rows (in
+// over K and V and a second launch; k_attn's time grows with the rows (in
 // blocks of 32 per KV head), the keys and the head_dim.  Both measured, us a
 // call with host work (k_attn / packed), by that product:
-//   59e6   32 rows of 32/8 heads of 128, 449 keys        50 / 50
-//   118e6  64 rows of the same                           52 / 50
-//   134e6  16 rows, 2042 keys                            57 / 58
-//   150e6  3 x 16 rows of 12 heads of 64, 2042 keys      61 / 62
-//   200e6  64 rows of 16/2 heads of 96, 2042 keys        86 / 46
-//   268e6  32 rows of 32/8 heads of 128, 2042 keys       92 / 58
-//   401e6  3 x 16 rows of 16 heads of 128, 2042 keys    143 / 105
-// head_dim 32 and below stays with k_attn: there its error is the smaller one
-// (2.4e-7 against 3.0e-7).
+//   59e6   32 rows of 32/8 heads of 128, 449 keys        48 / 47
+//   118e6  64 rows of the same                           49 / 48
+//   134e6  16 rows, 2042 keys                            55 / 53
+//   150e6  3 x 16 rows of 12 heads of 64, 2042 keys      59 / 57
+//   200e6  64 rows of 16/2 heads of 96, 2042 keys        82 / 41
+//   268e6  32 rows of 32/8 heads of 128, 2042 keys       88 / 52
+//   401e6  3 x 16 rows of 16 heads of 128, 2042 keys    141 / 95
+// Below the line the two are within 2 us; k_attn needs no scratch there.
+// head_dim 32 and below stays with k_attn, whose error was the smaller one
+// (2.4e-7 against 3.0e-7 with lo unscaled).
 extern "C" int cgk_attn_prompt_pays(int B, int Nq, int Nk, int H, int Hk, int D) {
     const double rows = ((long long)((H + Hk - 1) / Hk) * Nq + 31) / 32 * 32.0;
     return D > 32 && D <= 128 && (double)B * Hk * rows * Nk * D >= 1e6 * g_min_mega;
@@ -663,13 +644,9 @@ extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* 
     PromptArgs a;
     memset(&pk, 0, sizeof(pk));
     memset(&a, 0, sizeof(a));
-    // rows per block: 64, or 128 (a record in LDS serves twice the rows) up to
-    // head_dim 64, where the registers allow it, once that still gives two
-    // blocks a CU; key splits until there are two blocks a CU, of at least 8
-    // tiles each
-    const long long b64 = (R + 63) / 64 * Hk * B;
-    const int RT = DP <= 64 && b64 >= 1024 ? 2 : 1;
-    const long long chunks = (R + 64 * RT - 1) / (64 * RT), blocks = chunks * Hk * B;
+    // 64 rows a block; key splits until there are two blocks a CU, of at least
+    // 8 tiles each
+    const long long chunks = (R + 63) / 64, blocks = chunks * Hk * B;
     long long splits = 512 / blocks;
     if (splits > tiles / 8) splits = tiles / 8;
     if (splits < 1) splits = 1;
@@ -708,8 +685,8 @@ extern "C" int cgk_attn_prompt_f32(const float* Q, const float* K, const float* 
     a.vec = D == DP && !((uintptr_t)O & 15);
     a.O = O;
     a.lse = lse;
-    const int rc = DP == 64 ? launch_all<64>(pk, a, RT)
-                 : DP == 96 ? launch_all<96>(pk, a, RT) : launch_all<128>(pk, a, RT);
+    const int rc = DP == 64 ? launch_all<64>(pk, a)
+                 : DP == 96 ? launch_all<96>(pk, a) : launch_all<128>(pk, a);
     if (rc || splits == 1) return rc;
     return cgk_attn_combine(a.part_o, a.part_ml, (int)splits, (int)nrow, D, Nq, H, O, lse);
 }

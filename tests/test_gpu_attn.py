@@ -561,6 +561,35 @@ def test_flash_packed_far_exponents(gpu, rng, packed_always, eq, ek, ev):
     check_packed(gpu, Q, K, V, 1)
 
 
+@pytest.mark.parametrize("D", [64, 100, 128])
+def test_flash_packed_small_dims_keep_their_bits(gpu, rng, packed_always, D):
+    # dims of V down to 2^-30 of their row's largest, and Q and K of opposite
+    # slopes whose products all count: an operand is off by at most 2^-23 of
+    # itself or 2^-52 of its row's maximum, so every dim of O is held to its own
+    # size
+    Q, K, V = attn_inputs(rng, 1, 70, 150, 4, 2, D)
+    e = np.exp2(np.round(np.linspace(0, 30, D))).astype(np.float32)
+    Q, K, V = Q * e, K / e, V / rng.permutation(e)
+    O, _, p = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, 1, 0, None)
+    eO, _ = attention64(Q, K, V, p.scale, 1)
+    err = np.abs(O - eO).max(axis=(0, 1)) / np.abs(eO).max(axis=(0, 1))
+    assert err.max() <= PACKED_TOL
+
+
+def test_flash_packed_small_weights_keep_their_bits(gpu, rng, packed_always):
+    # V is the unit matrix: O holds the weights, each to its own size down to
+    # 2^-28 of the row's largest (2^-49 of it over the weight, and a score's
+    # error of 15 times 2^-21)
+    Q, K, _ = attn_inputs(rng, 1, 64, 64, 2, 2, 64)
+    V = np.broadcast_to(np.eye(64, dtype=np.float32)[None, :, None], (1, 64, 2, 64)).copy()
+    Q *= np.float32(3)
+    O, _, p = run_flash(gpu, "cg_flash_attention_forward", Q, K, V, 0, 0, None)
+    eO, _ = attention64(Q, K, V, p.scale, 0)
+    seen = eO >= 2.0 ** -28 * eO.max(-1, keepdims=True)
+    assert seen.any(where=eO < 2.0 ** -20) and np.all(O >= 0)
+    assert np.max(np.abs(O - eO)[seen] / eO[seen]) <= 1e-5
+
+
 @pytest.mark.parametrize("where", ["q", "k", "v"])
 def test_flash_packed_non_finite_inputs(gpu, rng, where):
     # infinities and NaN give what the fp32 kernel gives, bit for bit, and
