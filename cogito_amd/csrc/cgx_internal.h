@@ -43,6 +43,10 @@ typedef struct {
     int K, N, group_size;
     int paired;          /* layout 3: gate|up tiles interleaved (SwiGLU) */
     float smax;          /* layout 3: max |scale| (the GEMM's row-scaling bound) */
+    /* layout 3, scales too far apart for one row scaling of the GEMM: its own
+     * scales ([N/gs][K], cgk_int4_group_scales) and after them the groups'
+     * multipliers [N/gs]; else NULL */
+    float* group_scales;
 } cgx_qinfo;
 int cgx_quant_lookup(const cg_tensor_quant* q, cgx_qinfo* info);
 void cgx_quant_register(const cg_tensor_quant* q, const cgx_qinfo* info);
@@ -89,13 +93,20 @@ int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int gs, const ui
                   const float* scales_t, float smax, float* y, int ldy, int pro,
                   const float* nw, float eps, int epi, const float* stats_in, int nstat_in,
                   float* stats_out, const float* nw_next);
+/* Scales of layout 3 ([N/gs][K]) brought to a common range, below 2: each group
+ * of columns times a power of two whose inverse is up[g]; scales of all-zero
+ * nibbles count as zero.  cgk_group_mul multiplies the product over them, y
+ * [M][N], by its groups' up. */
+int cgk_int4_group_scales(const uint8_t* flat, const float* scales_t, int K, int N, int gs,
+                          float* out, float* up);
+int cgk_group_mul(float* y, int M, int N, int gs, const float* up);
 /* Dispatch of plain products between the GEMM and the GEMV: whether M rows
  * pay for the GEMM, the rows of one GEMM call, and whether its scratch is at
  * hand (not under stream capture). */
 int cgk_gemm_int4_pays(int M, int K, int N, int gs);
 int cgk_gemm_int4_max_rows(int K, int N);
 int cgk_gemm_int4_ready(int M, int K, int N, int gs);
-int cgk_absmax(const float* s, size_t n, float* out_host);
+int cgk_absrange(const float* s, size_t n, float* hi, float* lo);
 int cgk_gemv_mfma(const float* x, int ldx, int M, int K, int N, int gs, const uint8_t* w,
                   const float* scales_t, float* y, int ldy, int pro, const float* nw, float eps,
                   int epi);

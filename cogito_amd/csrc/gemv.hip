@@ -935,7 +935,10 @@ int launch_pe(const MfmaArgs& a, int T) {
 // scale of that slot's group at each k) times a per-row factor rstd * 2^E,
 // split into hi + lo fp16 (22 significant bits); the MFMA sums are scaled by
 // 2^-E at the end.  k_gemm_rows fixes the row factors before the GEMM from
-// the whole row: max|x * nw| * rstd * max|s| * 2^E < 2^15.  The next step's
+// the whole row: max|x * nw| * rstd * max|s| * 2^E < 2^15, so that an element
+// is off by at most 2^-22 of itself or 2^-39 of that bound (plain products over
+// scales too far apart for one bound take cgk_int4_group_scales').  The next
+// step's
 // activations and the weights two steps ahead are loaded while a step is
 // multiplied.  K is split over blockIdx.z; k_gemm_reduce sums the splits in
 // a fixed order and applies the epilogue (store, accumulate, SwiGLU of the
@@ -1888,32 +1891,102 @@ extern "C" int cgk_gemm_int4(const float* x, int ldx, int M, int K, int N, int g
     return launch_check("k_gemm_reduce");
 }
 
-// max |s| over a scales array (host result, synchronising)
-__global__ void k_absmax(const float* __restrict__ s, size_t n, unsigned int* out) {
-    float m = 0.0f;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        m = fmaxf(m, fabsf(s[i]));
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));
+// y[m][col] *= up[col / gs], four outputs a thread.
+__global__ __launch_bounds__(256) void k_group_mul(float* __restrict__ y, unsigned n4, unsigned N4,
+                                                   unsigned gs4, const float* __restrict__ up) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const float u = up[i % N4 / gs4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) y[4 * (size_t)i + j] *= u;
 }
 
-extern "C" int cgk_absmax(const float* s, size_t n, float* out_host) {
-    unsigned int* d = (unsigned int*)cgx_scratch(CGX_SLOT_OUT1, 16);
+extern "C" int cgk_group_mul(float* y, int M, int N, int gs, const float* up) {
+    const unsigned n4 = (unsigned)((size_t)M * N / 4);      // M N < 2^31 (cgk_gemm_int4)
+    hipLaunchKernelGGL(k_group_mul, dim3((n4 + 255) / 256), dim3(256), 0, stream(), y, n4,
+                       (unsigned)N / 4, (unsigned)gs / 4, up);
+    return launch_check("k_group_mul");
+}
+
+// Scales for the GEMM of a weight whose scales lie far apart: those of a group
+// of columns times the power of two that brings its largest into [1, 2), and
+// its inverse in up[g].  A scale whose nibbles all are zero (the quantiser gives
+// such a group scale 1) counts as zero: it would set the bound for nothing.  One
+// block per group.
+__global__ __launch_bounds__(256) void k_group_scales(const uint8_t* __restrict__ flat,
+                                                      const float* __restrict__ scales_t, int K,
+                                                      int N, int gs, float* __restrict__ out,
+                                                      float* __restrict__ up) {
+    __shared__ float s_m[4];
+    const int g = blockIdx.x;
+    float m = 0.0f;
+    for (int k = threadIdx.x; k < K; k += 256) {
+        const uint8_t* p = flat + ((size_t)k * N + (size_t)g * gs) / 2;
+        unsigned any = 0;
+        for (int i = 0; i < gs / 2; i++) any |= p[i];
+        const float s = any ? scales_t[(size_t)g * K + k] : 0.0f;
+        out[(size_t)g * K + k] = s;
+        m = fmaxf(m, fabsf(s));
+    }
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3]));
+    int e = m > 0.0f && m < __builtin_inff() ? ilogbf(m) : 0;
+    e = e < -120 ? -120 : e;              // 2^e is no subnormal
+    for (int k = threadIdx.x; k < K; k += 256)      // (the elements this thread wrote)
+        out[(size_t)g * K + k] = ldexpf(out[(size_t)g * K + k], -e);
+    if (threadIdx.x == 0) up[g] = ldexpf(1.0f, e);
+}
+
+extern "C" int cgk_int4_group_scales(const uint8_t* flat, const float* scales_t, int K, int N,
+                                     int gs, float* out, float* up) {
+    hipLaunchKernelGGL(k_group_scales, dim3(N / gs), dim3(256), 0, stream(), flat, scales_t, K, N,
+                       gs, out, up);
+    return launch_check("k_group_scales");
+}
+
+// Largest and smallest non-zero |s| over a scales array (host results,
+// synchronising; no scale but zeros: 0 and infinity): a pair a block, finished
+// on the host.
+constexpr int kRangeBlocks = 256;
+
+__global__ __launch_bounds__(256) void k_absrange(const float* __restrict__ s, size_t n,
+                                                  float2* __restrict__ out) {
+    __shared__ float2 lds[4];
+    float hi = 0.0f, lo = __builtin_inff();
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += kRangeBlocks * 256) {
+        const float v = fabsf(s[i]);
+        hi = fmaxf(hi, v);
+        if (v > 0.0f) lo = fminf(lo, v);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        hi = fmaxf(hi, __shfl_xor(hi, o));
+        lo = fminf(lo, __shfl_xor(lo, o));
+    }
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = make_float2(hi, lo);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; w++) {
+            hi = fmaxf(hi, lds[w].x);
+            lo = fminf(lo, lds[w].y);
+        }
+        out[blockIdx.x] = make_float2(hi, lo);
+    }
+}
+
+extern "C" int cgk_absrange(const float* s, size_t n, float* hi, float* lo) {
+    float2 r[kRangeBlocks];
+    float2* d = (float2*)cgx_scratch(CGX_SLOT_OUT1, sizeof r);
     if (!d) return -1;
-    unsigned int zero = 0u, r = 0u;
-    if (hipMemcpyAsync(d, &zero, 4, hipMemcpyHostToDevice, stream()) != hipSuccess) {
-        cgx_set_error("absmax: copy failed");
-        return -1;
+    hipLaunchKernelGGL(k_absrange, dim3(kRangeBlocks), dim3(256), 0, stream(), s, n, d);
+    if (launch_check("k_absrange") || cgx_memcpy_d2h(r, d, sizeof r)) return -1;
+    float h = 0.0f, l = __builtin_inff();
+    for (const float2& v : r) {
+        h = v.x > h ? v.x : h;
+        l = v.y < l ? v.y : l;
     }
-    hipLaunchKernelGGL(k_absmax, dim3(256), dim3(256), 0, stream(), s, n, d);
-    if (launch_check("k_absmax")) return -1;
-    if (hipMemcpyAsync(&r, d, 4, hipMemcpyDeviceToHost, stream()) != hipSuccess ||
-        hipStreamSynchronize(stream()) != hipSuccess) {
-        cgx_set_error("absmax: copy failed");
-        return -1;
-    }
-    float f;
-    memcpy(&f, &r, sizeof f);
-    *out_host = f;
+    *hi = h;
+    if (lo) *lo = l;
     return 0;
 }

@@ -246,7 +246,7 @@ static int make_lin(cgx_model* m, lin_t* L, int which, int layer, float* tf, uin
     if (cgk_int4_repack_mfma(tq, ts, L->K, L->N, m->c.group_size, which == W_GU, L->tiled,
                              L->scales_t))
         return -1;
-    return cgk_absmax(L->scales_t, n / m->c.group_size, &L->smax);
+    return cgk_absrange(L->scales_t, n / m->c.group_size, &L->smax, NULL);
 }
 
 static void free_lin(lin_t* L) {

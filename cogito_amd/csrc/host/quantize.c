@@ -95,6 +95,16 @@ static int quant_dims(const cg_tensor_quant* q, int* K, int* N) {
     return (*K) * (*N) == q->size ? 0 : -1;
 }
 
+/* The GEMM scales a row of x by one power of two, from the weight's largest
+ * scale; the GEMV by one per 256 rows of W and scale group.  A group of columns
+ * whose scales lie far below the largest loses bits in the GEMM (error of the
+ * group against 64 bits, 64 x 4096: 1.6e-7 of it up to a ratio of 2^13, 1.8e-7
+ * at 2^14, 3.5e-7 at 2^16, 5.3e-6 at 2^20; in the GEMV 2.0e-7 throughout).
+ * Weights of a wider range keep a second copy of their scales for the GEMM,
+ * each group of columns in a range of its own, and take a pass over the product
+ * that multiplies the groups' ranges back. */
+#define GEMM_SCALE_RANGE 16384.0f
+
 static cg_tensor_quant* quant_to_device_layout(cg_tensor_quant* q, int want) {
     if (!q || !q->data || !q->scales || q->size <= 0 || q->group_size <= 0) {
         cgx_set_error("cgx_quant_to_device: invalid quantized tensor");
@@ -129,6 +139,7 @@ static cg_tensor_quant* quant_to_device_layout(cg_tensor_quant* q, int want) {
         return NULL;
     }
     memcpy(d->shape, q->shape, (size_t)q->ndim * sizeof(int));
+    cgx_qinfo info = {layout, K, N, gs, 0, 0.0f, NULL};
     d->data = (uint8_t*)cgx_malloc(nb);
     d->scales = (float*)cgx_malloc((size_t)ng * 4);
     if (!d->data || !d->scales) goto fail;
@@ -140,7 +151,20 @@ static cg_tensor_quant* quant_to_device_layout(cg_tensor_quant* q, int want) {
                 ? cgk_int4_repack_mfma(fd, fs, K, N, gs, 0, d->data, d->scales)
                 : cgk_int4_repack_tiled(fd, fs, K, N, gs, d->data, d->scales))
             goto fail;
-        if (cgx_synchronize()) goto fail;
+        if (layout != CGX_LAYOUT_MFMA) {
+            if (cgx_synchronize()) goto fail;
+        } else {                          /* (the range waits for the repack) */
+            float smin = 0.0f;
+            if (cgk_absrange(d->scales, (size_t)ng, &info.smax, &smin)) goto fail;
+            if (!(info.smax <= GEMM_SCALE_RANGE * smin)) {
+                info.group_scales = (float*)cgx_malloc(((size_t)ng + N / gs) * 4);
+                if (!info.group_scales ||
+                    cgk_int4_group_scales(fd, d->scales, K, N, gs, info.group_scales,
+                                          info.group_scales + ng) ||
+                    cgx_synchronize())
+                    goto fail;
+            }
+        }
     } else {
         int dev = cgx_is_device_ptr(q->data);
         if ((dev ? cgx_memcpy_d2d(d->data, q->data, nb)
@@ -150,13 +174,10 @@ static cg_tensor_quant* quant_to_device_layout(cg_tensor_quant* q, int want) {
             cgx_synchronize())
             goto fail;
     }
-    {
-        cgx_qinfo info = {layout, K, N, gs, 0, 0.0f};
-        if (layout == CGX_LAYOUT_MFMA && cgk_absmax(d->scales, (size_t)ng, &info.smax)) goto fail;
-        cgx_quant_register(d, &info);
-    }
+    cgx_quant_register(d, &info);
     return d;
 fail:
+    cgx_free(info.group_scales);
     cgx_free(d->data);
     cgx_free(d->scales);
     free(d->shape);
@@ -188,8 +209,10 @@ int cgx_quant_layout(cg_tensor_quant* q) {
 
 void cg_tensor_quant_free(cg_tensor_quant* q) {
     if (!q) return;
-    if (cgx_quant_lookup(q, NULL)) {
+    cgx_qinfo info;
+    if (cgx_quant_lookup(q, &info)) {
         cgx_quant_unregister(q);
+        cgx_free(info.group_scales);
         cgx_free(q->data);
         cgx_free(q->scales);
         free(q->shape);
@@ -253,14 +276,19 @@ static int matmul_mfma(const float* x, int M, const cg_tensor_quant* w, const cg
                        float* y) {
     const int K = info->K, N = info->N, gs = info->group_size;
     const int most = cgk_gemm_int4_max_rows(K, N);
+    const float* gs_t = info->group_scales ? info->group_scales : w->scales;
+    const float* up = info->group_scales ? gs_t + (size_t)K * (N / gs) : NULL;
     for (int m0 = 0; m0 < M;) {
         const int rows = M - m0 < most ? M - m0 : most;
         const float* xr = x + (size_t)m0 * K;
         float* yr = y + (size_t)m0 * N;
         int rc;
         if (cgk_gemm_int4_pays(rows, K, N, gs) && cgk_gemm_int4_ready(rows, K, N, gs))
-            rc = cgk_gemm_int4(xr, K, rows, K, N, gs, w->data, w->scales, info->smax, yr, N, 0,
-                               NULL, 0.0f, 0, NULL, 0, NULL, NULL);
+            rc = cgk_gemm_int4(xr, K, rows, K, N, gs, w->data, gs_t, up ? 2.0f : info->smax, yr, N,
+                               0, NULL, 0.0f, 0, NULL, 0, NULL, NULL) ||
+                         (up && cgk_group_mul(yr, rows, N, gs, up))
+                     ? -1
+                     : 0;
         else
             rc = cgk_gemv_mfma(xr, K, rows, K, N, gs, w->data, w->scales, yr, N, 0, NULL, 0.0f,
                                0);

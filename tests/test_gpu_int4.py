@@ -154,6 +154,50 @@ def test_matmul_many_rows_wide_dynamic_range(gpu, oracle, rng):
     gpu.cg_tensor_quant_free(dq)
 
 
+def _gemv64(x, data, scales, K, N, gs):
+    w = np.empty(K * N, np.int8)
+    w[0::2], w[1::2] = data & 15, data >> 4
+    w = np.where(w > 7, w - 16, w).astype(np.float64).reshape(K, N)
+    return x.astype(np.float64) @ (w * np.repeat(scales.reshape(K, N // gs), gs, 1))
+
+
+@pytest.mark.parametrize("gs", [128, 64, 32])
+@pytest.mark.parametrize("kind", ["column group", "zero groups", "infinite scale"])
+def test_matmul_many_rows_scales_far_apart(gpu, rng, kind, gs):
+    """Columns whose scales lie far below the weight's largest keep their bits:
+    each scale group is held to its own size.  A product of the split operands
+    is off by 2^-22 of itself, sums of 1024 by a few 2^-24."""
+    print(f"scales far apart: {kind}, groups of {gs}", flush=True)
+    K, N, M, tol = 1024, 512, 64, 3e-6
+    data = rng.integers(0, 256, K * N // 2, dtype=np.uint8)
+    scales = rng.uniform(0.005, 0.02, (K, N // gs)).astype(np.float32)
+    ok = np.ones(N // gs, bool)
+    if kind == "column group":
+        scales[:, 1::2] *= np.float32(1e-8)
+    elif kind == "zero groups":            # scale 1 by the quantiser's rule
+        scales *= np.float32(1e-7)
+        scales[5] = scales[700, ::2] = scales[:, 1] = 1.0
+        nib = data.reshape(K, N // gs, gs // 2)
+        nib[5] = 0
+        nib[700, ::2] = nib[:, 1] = 0
+        ok[1] = False
+    else:
+        scales[3, 0] = np.inf
+        ok[0] = False
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    ref = _gemv64(x, data, np.where(np.isinf(scales), 0, scales), K, N, gs)
+    hq, keep = host_quant_from_arrays(data, scales.ravel(), K, N, gs)
+    dq = gpu.cgx_quant_to_device_layout(C.byref(hq), 3)
+    dx, dy = DeviceArray.from_numpy(gpu, x), DeviceArray(gpu, M * N * 4)
+    assert gpu.cgx_matmul_int4_dev(dx.ptr, M, dq, dy.ptr) == 0, last_error(gpu)
+    assert gpu.cgx_synchronize() == 0
+    y = dy.numpy(np.float32, (M, N // gs, gs))[:, ok]
+    ref = ref.reshape(M, N // gs, gs)[:, ok]
+    err = np.abs(y - ref).max(axis=(0, 2)) / np.abs(ref).max(axis=(0, 2))
+    assert err.max() <= tol, err
+    gpu.cg_tensor_quant_free(dq)
+
+
 def test_matmul_many_rows_under_capture(gpu, rng):
     # a captured product takes the path without scratch memory: every replay
     # on new inputs equals the eager GEMV, with larger eager products (which
