@@ -7,14 +7,13 @@
  * h * n_heads_k / n_heads (reference src/cuda/flash_attn_kernels.c:278).
  *
  * MI355X implementation: cg_flash_attention_forward (and its _cpu-named
- * twin, kept for source compatibility) run a HIP split-KV flash kernel on
- * the GPU.  Mask types:
+ * twin, kept for source compatibility) run on the GPU: a split-KV flash
+ * kernel over fp32 operands, or for larger calls of head_dim 33 to 128 one
+ * over K and V packed into fp16 hi + lo pairs.  Mask types:
  *   ATTN_MASK_NONE, ATTN_MASK_SLIDING_WINDOW -- as the reference;
- *   ATTN_MASK_CAUSAL -- bottom-right aligned: query i sees keys
- *     [0, seqlen_k - seqlen_q + i].  For seqlen_q == seqlen_k this is the
- *     reference's rule (k_idx > q_idx masked, src/attention/flash_attn.c:82);
- *     for verify (seqlen_q < seqlen_k) the reference rule would mask the
- *     cached context, so the aligned form is used;
+ *   ATTN_MASK_CAUSAL -- as the reference: query i sees keys [0, i]
+ *     (k_idx > q_idx masked, src/attention/flash_attn.c:82), whatever
+ *     seqlen_k;
  *   ATTN_MASK_CUSTOM -- `mask` is an additive fp32 [seqlen_q, seqlen_k] mask
  *     (e.g. the rows of cg_tree_attention_mask for the new tokens).
  * Backward passes are training-only and not provided (set the last error).

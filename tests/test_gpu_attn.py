@@ -126,7 +126,7 @@ def test_kv_write_block_and_device_get(gpu, oracle, rng):
 def test_kv_write_get_forms(gpu, oracle, rng, H, D, gs, T, pos, off):
     # groups of one lane to a whole wave, of a count of lanes that is no power
     # of two, of less than a unit; rows off the 16-byte line (`off` floats);
-    # ragged lengths; zeros, infinities and values at the rounding's halves
+    # ragged lengths; zeros and values at the rounding's halves
     S = pos + T
     k = rng.normal(0, 1, (S, H, D)).astype(np.float32)
     v = rng.normal(0, 2, (S, H, D)).astype(np.float32)
@@ -467,11 +467,12 @@ def test_flash_packed_vs_oracle(gpu, oracle, rng, packed_always, B, Nq, Nk, H, H
     fin = else_ > -1e30
     np.testing.assert_allclose(lse[fin], else_[fin], rtol=1e-4, atol=1e-4)
     assert np.all(lse[~fin] == else_[~fin])
+    check_packed(gpu, Q, K, V, mt, W, mask)         # and to the operands' bits
 
 
 def test_flash_packed_magnitudes(gpu, oracle, rng, packed_always):
-    # rows of Q, K and V many binades apart (the products in fp32's range):
-    # every row keeps its own scale
+    # rows of K and V many binades apart (the products in fp32's range): every
+    # row keeps its own scale
     Q, K, V = attn_inputs(rng, 1, 40, 90, 4, 2, 64)
     e = lambda n, h: np.exp2(rng.integers(-40, 40, (1, n, h, 1))).astype(np.float32)
     ek = e(90, 2)

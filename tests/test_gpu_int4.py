@@ -161,6 +161,52 @@ def _gemv64(x, data, scales, K, N, gs):
     return x.astype(np.float64) @ (w * np.repeat(scales.reshape(K, N // gs), gs, 1))
 
 
+# of a scale group's largest output, in a row: an operand of the GEMM is off by
+# at most 2^-22 of itself (2.4e-7), the sums of up to 11008 products by less than
+# ten times that; without the lo halves the error is 2^-11
+GEMM_TOL = 3e-6
+
+
+def check_groups(gpu, x, data, scales, K, N, gs):
+    """The default dispatch against 64 bits, each scale group of a row held to
+    its own largest value."""
+    M = x.shape[0]
+    hq, keep = host_quant_from_arrays(data, scales.ravel(), K, N, gs)
+    dq = gpu.cgx_quant_to_device_layout(C.byref(hq), 3)
+    dx, dy = DeviceArray.from_numpy(gpu, x), DeviceArray(gpu, M * N * 4)
+    assert gpu.cgx_matmul_int4_dev(dx.ptr, M, dq, dy.ptr) == 0, last_error(gpu)
+    assert gpu.cgx_synchronize() == 0
+    y = dy.numpy(np.float32, (M, N // gs, gs))
+    ref = _gemv64(x, data, scales, K, N, gs).reshape(M, N // gs, gs)
+    err = np.abs(y - ref).max(axis=2) / np.abs(ref).max(axis=2)
+    assert err.max() <= GEMM_TOL, err.max()
+    gpu.cg_tensor_quant_free(dq)
+
+
+@pytest.mark.parametrize("K,N,gs,M", [
+    (256, 128, 128, 49), (768, 3072, 128, 97), (4096, 4096, 128, 25), (11008, 1024, 128, 70),
+    (1024, 640, 128, 65), (512, 768, 256, 50), (256, 96, 32, 49), (768, 704, 64, 97),
+    (512, 864, 96, 64), (4096, 2048, 32, 60), (4096, 2048, 64, 60)])
+def test_matmul_many_rows_against_64_bits(gpu, rng, K, N, gs, M):
+    print(f"GEMM against 64 bits M={M} K={K} N={N} gs={gs}", flush=True)
+    data = rng.integers(0, 256, K * N // 2, dtype=np.uint8)
+    scales = rng.uniform(0.005, 0.02, (K, N // gs)).astype(np.float32)
+    check_groups(gpu, rng.normal(0, 1, (M, K)).astype(np.float32), data, scales, K, N, gs)
+
+
+@pytest.mark.parametrize("gs", [128, 32])
+def test_matmul_many_rows_rows_and_groups_far_apart(gpu, rng, gs):
+    # rows up to 2^80 and groups of columns up to 2^40 apart, each pair to its
+    # own size
+    print(f"rows and groups far apart, groups of {gs}", flush=True)
+    K, N, M = 1024, 512, 64
+    data = rng.integers(0, 256, K * N // 2, dtype=np.uint8)
+    scales = rng.uniform(0.005, 0.02, (K, N // gs))
+    scales = (scales * np.exp2(rng.integers(-20, 21, N // gs))).astype(np.float32)
+    x = rng.normal(0, 1, (M, K)) * np.exp2(rng.integers(-40, 41, (M, 1)))
+    check_groups(gpu, x.astype(np.float32), data, scales, K, N, gs)
+
+
 @pytest.mark.parametrize("gs", [128, 64, 32])
 @pytest.mark.parametrize("kind", ["column group", "zero groups", "infinite scale"])
 def test_matmul_many_rows_scales_far_apart(gpu, rng, kind, gs):
