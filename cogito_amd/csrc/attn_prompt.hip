@@ -33,8 +33,9 @@
 // ends early; tiles that no row of the block sees are skipped.  Measured at
 // that size: 724 us for k_attn (scalar K loads a row apart, every tile of the
 // causal mask), 80 us for the call here.  A call whose inputs the operands
-// cannot hold costs this time before k_attn's.  The VALU's share bounds it:
-// about 175 instructions a wave and tile beside 48 MFMAs.
+// cannot hold costs this time before k_attn's.  Waiting bounds it, two waves a
+// SIMD that meet at a barrier every tile: 238 vector instructions a wave and
+// tile beside 48 MFMAs keep the VALU 25 % and the matrix cores 16 % busy.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>

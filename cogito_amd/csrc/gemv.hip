@@ -938,9 +938,8 @@ int launch_pe(const MfmaArgs& a, int T) {
 // the whole row: max|x * nw| * rstd * max|s| * 2^E < 2^15, so that an element
 // is off by at most 2^-22 of itself or 2^-39 of that bound (plain products over
 // scales too far apart for one bound take cgk_int4_group_scales').  The next
-// step's
-// activations and the weights two steps ahead are loaded while a step is
-// multiplied.  K is split over blockIdx.z; k_gemm_reduce sums the splits in
+// step's activations and the weights two steps ahead are loaded while a step
+// is multiplied.  K is split over blockIdx.z; k_gemm_reduce sums the splits in
 // a fixed order and applies the epilogue (store, accumulate, SwiGLU of the
 // gate|up pair).
 //
@@ -960,7 +959,7 @@ constexpr int kGemmRowH = kChunkK + 8;   // LDS pitch (halfs) of an A row
 // values and are then added to the split's sums, so that few roundings happen
 // at a long sum's full magnitude (error against 64 bits, 4096 x 11008 at 509
 // rows: 4.7e-7 of the result in one chain, 1.9e-7 folded, 2.0e-7 in the GEMV;
-// for 3 % of the time, 114 -> 118 us).  Plain products only: the decoder's
+// for 3 % of the time).  Plain products only: the decoder's
 // layers keep one chain (two layers of the 7B shape at 256 rows: 610 us in one
 // chain, 644 folded).
 constexpr int kGemmFold = 4;
